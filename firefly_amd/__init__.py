@@ -74,6 +74,11 @@ def _load() -> ctypes.CDLL:
     lib.ffkv_paged_prefill.restype = i32
     lib.ffkv_paged_prefill.argtypes = [vp, vp, i32, vp, vp, i32, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32,
                                        i32, i32, ctypes.c_float, vp]
+    lib.ffkv_prefill_workspace_bytes.restype = sz
+    lib.ffkv_prefill_workspace_bytes.argtypes = [i32] * 10
+    lib.ffkv_paged_prefill_ws.restype = i32
+    lib.ffkv_paged_prefill_ws.argtypes = [vp, vp, i32, vp, vp, i32, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32,
+                                          i32, i32, f32, vp, sz, vp]
     lib.ffkv_rope.restype = i32
     lib.ffkv_rope.argtypes = [vp, vp, i32, vp, i32, i32, i32, i32, i32, ctypes.c_float, vp]
     lib.ffkv_rope_append.restype = i32
@@ -154,11 +159,32 @@ def paged_prefill(q, k_cache, v_cache, block_table, context_lens, out=None, k_sc
         out = torch.empty((B, S, Hq * D), dtype=q.dtype, device=q.device)
     max_blocks = 0 if block_table is None else block_table.shape[-1]
     N = (k_cache.shape[0] if num_blocks is None else num_blocks) if block_table is not None else 0
-    check(lib.ffkv_paged_prefill(_ptr(q), _ptr(out), torch_dtype_code(q), _ptr(k_cache), _ptr(v_cache),
-                                 torch_dtype_code(k_cache), _ptr(k_scale), _ptr(v_scale), _ptr(block_table),
-                                 _ptr(context_lens), B, S, Hq, Hkv, D, BLOCK_SIZE, max_blocks, N, max_context_len,
-                                 float(scale), _stream(stream)))
+    qt, ct = torch_dtype_code(q), torch_dtype_code(k_cache)
+    ws, ws_bytes = _prefill_scratch(lib.ffkv_prefill_workspace_bytes(qt, ct, B, S, Hq, Hkv, D, block_table is not None,
+                                                                     max_blocks, max_context_len), q.device, stream)
+    check(lib.ffkv_paged_prefill_ws(_ptr(q), _ptr(out), qt, _ptr(k_cache), _ptr(v_cache), ct, _ptr(k_scale),
+                                    _ptr(v_scale), _ptr(block_table), _ptr(context_lens), B, S, Hq, Hkv, D, BLOCK_SIZE,
+                                    max_blocks, N, max_context_len, float(scale), _ptr(ws), ws_bytes,
+                                    _stream(stream)))
     return out
+
+
+def _prefill_scratch(n: int, device, stream):
+    """Scratch of ``n`` bytes for one call on ``stream`` (None: the current one), from torch's allocator and belonging
+    to that stream, so that it can be reused once the call's work on the stream is done.  None while the stream is
+    being captured (a capture allocates nothing here; the call then runs unsplit)."""
+    import torch
+
+    if n == 0:
+        return None, 0
+    if stream is not None:
+        if not isinstance(stream, torch.cuda.Stream):
+            stream = torch.cuda.ExternalStream(int(getattr(stream, "cuda_stream", stream)), device=device)
+        with torch.cuda.stream(stream):
+            return _prefill_scratch(n, device, None)
+    if torch.cuda.is_current_stream_capturing():
+        return None, 0
+    return torch.empty(n, dtype=torch.uint8, device=device), n
 
 
 def apply_rope(q, k, context_lens=None, theta: float = 1e6, stream=None) -> None:

@@ -251,6 +251,40 @@ int ffkv_paged_prefill(const void* q, void* out, int qo_dtype, const void* k_cac
                        int head_dim, int block_size, int max_blocks, int num_blocks, int max_context_len, float scale,
                        void* stream)
 {
+    return ffkv_paged_prefill_ws(q, out, qo_dtype, k_cache, v_cache, cache_dtype, k_scale, v_scale, block_table,
+                                 context_lens, batch, seq_len, num_heads, num_kv_heads, head_dim, block_size,
+                                 max_blocks, num_blocks, max_context_len, scale, nullptr, 0, stream);
+}
+
+size_t ffkv_prefill_workspace_bytes(int qo_dtype, int cache_dtype, int batch, int seq_len, int num_heads,
+                                    int num_kv_heads, int head_dim, int paged, int max_blocks, int max_context_len)
+{
+    // sizes that ffkv_paged_prefill refuses need nothing
+    if (!is_act(qo_dtype) || !is_cache(cache_dtype) || cache_dtype == FFKV_DTYPE_F32 || !head_dim_mfma(head_dim) ||
+        batch <= 0 || batch > 65535 || seq_len <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_kv_heads > 65535 ||
+        num_heads % num_kv_heads != 0 || (paged != 0 && max_blocks < 0))
+        return 0;
+    ffkv::PrefillArgs a{};
+    a.qo_dtype = qo_dtype;
+    a.cache_dtype = cache_dtype;
+    a.batch = batch;
+    a.seq_len = seq_len;
+    a.num_heads = num_heads;
+    a.num_kv_heads = num_kv_heads;
+    a.group = num_heads / num_kv_heads;
+    a.head_dim = head_dim;
+    a.paged = paged != 0;
+    a.cap_tokens = a.paged ? ffkv::decode_cap_tokens(max_blocks, max_context_len) : seq_len;
+    ffkv::prefill_plan(a);
+    return static_cast<size_t>(ffkv::prefill_split_layout(a).total);
+}
+
+int ffkv_paged_prefill_ws(const void* q, void* out, int qo_dtype, const void* k_cache, const void* v_cache,
+                          int cache_dtype, const float* k_scale, const float* v_scale, const int32_t* block_table,
+                          const int32_t* context_lens, int batch, int seq_len, int num_heads, int num_kv_heads,
+                          int head_dim, int block_size, int max_blocks, int num_blocks, int max_context_len,
+                          float scale, void* workspace, size_t workspace_bytes, void* stream)
+{
     const bool paged = block_table != nullptr;
     if (block_size != FFKV_BLOCK_SIZE) return fail(FFKV_ERR_UNSUPPORTED, "block_size must be 16, got %d", block_size);
     if (!is_act(qo_dtype)) return fail(FFKV_ERR_UNSUPPORTED, "unsupported q/out dtype %d", qo_dtype);
@@ -304,6 +338,24 @@ int ffkv_paged_prefill(const void* q, void* out, int qo_dtype, const void* k_cac
     a.cap_tokens = paged ? ffkv::decode_cap_tokens(max_blocks, max_context_len) : seq_len;
     a.paged = paged;
     a.scale_log2 = sm_scale * 1.4426950408889634f;
+    a.n_split = 1;
+    if (workspace != nullptr)
+    {
+        if (!aligned16(workspace)) return fail(FFKV_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
+        ffkv::prefill_plan(a);
+        const ffkv::PrefillSplitLayout lay = ffkv::prefill_split_layout(a);
+        if (a.n_split > 1 && workspace_bytes >= static_cast<size_t>(lay.total))
+        {
+            char* w = static_cast<char*>(workspace);
+            a.ws_pieces = reinterpret_cast<int32_t*>(w + lay.pieces);
+            a.ws_ml = reinterpret_cast<float*>(w + lay.ml);
+            a.ws_acc = reinterpret_cast<float*>(w + lay.acc);
+        }
+        else
+        {
+            a.n_split = 1;
+        }
+    }
     hipError_t e = ffkv::launch_prefill(a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "prefill launch");
     return ok();

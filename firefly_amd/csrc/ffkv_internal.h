@@ -85,6 +85,15 @@ struct PrefillArgs
     int            pfx_slot0;
     float*         ws_ml;
     float*         ws_acc;
+    // Prefill split over the keys (launch_prefill with n_split > 1): each block of 128 query rows takes up to n_split
+    // pieces of its steps (the kernel's own number of keys), written as partials to the workspace and merged by a
+    // second kernel.  Blocks of fewer than split_from steps stay whole; a piece has at least kPrefillSplitMin steps,
+    // and as many more as it takes for all the call's pieces to fill split_slots workgroups once.  n_split <= 1: no
+    // pieces, no workspace.
+    int            n_split;
+    int            split_slots;
+    int            split_from;
+    int32_t*       ws_pieces;  // [row blocks]: pieces of each
 };
 
 struct DecodeArgs
@@ -137,6 +146,14 @@ hipError_t launch_append(const AppendArgs& a, hipStream_t stream);
 hipError_t launch_rope_append(const RopeArgs& a, hipStream_t stream);      // rotate q/k, then append when k_cache set
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream);  // matrix-core prefill (16- and 8-bit caches)
 hipError_t launch_prefix_partials(const PrefillArgs& a, hipStream_t stream);  // shared-prefix decode partials
+// Sets n_split, split_slots and split_from of a prefill whose sizes and dtypes are set; the partials of a split
+// prefill take prefill_split_layout's bytes.
+void prefill_plan(PrefillArgs& a);
+struct PrefillSplitLayout
+{
+    int64_t pieces, ml, acc, total;  // byte offsets of the three regions and their end (0: no split)
+};
+PrefillSplitLayout prefill_split_layout(const PrefillArgs& a);
 hipError_t launch_decode(const DecodeArgs& a, hipStream_t stream);       // generic kernel (any cache dtype)
 hipError_t launch_decode_mfma(const DecodeArgs& a, hipStream_t stream);  // matrix-core kernel (16-bit/8-bit caches)
 // Copies the first `width` ints of `rows` rows of `pitch` ints from src (pinned host memory mapped into the device's

@@ -186,10 +186,15 @@ void prefill(Tensor& q, Tensor& k, Tensor& v, const float* k_scale, const float*
         return fail("attention (prefill): k/v must be [.., .., kv_head_num, head_dim] and alike");
     if (block_table == nullptr && (k.shape()[0] != B || k.shape()[1] != S))
         return fail("attention (prefill): contiguous k/v must be [B, seq_len, kv_head_num, head_dim]");
-    const int rc = ffkv_paged_prefill(q.data(), out.data(), code(q.dtype()), k.data(), v.data(), code(k.dtype()),
-                                      k_scale, v_scale, reinterpret_cast<const int32_t*>(block_table), context_lens, B,
-                                      S, Hq, kv_head_num, D, FFKV_BLOCK_SIZE, block_table ? max_context_blocks : 0,
-                                      block_table ? static_cast<int>(k.shape()[0]) : 0, 0, 0.0f, t_stream);
+    const size_t need = ffkv_prefill_workspace_bytes(code(q.dtype()), code(k.dtype()), B, S, Hq, kv_head_num, D,
+                                                     block_table != nullptr, max_context_blocks, 0);
+    size_t       have = 0;
+    void*        ws = need > 0 ? workspace(need, have) : nullptr;
+    const int    rc = ffkv_paged_prefill_ws(
+        q.data(), out.data(), code(q.dtype()), k.data(), v.data(), code(k.dtype()), k_scale, v_scale,
+        reinterpret_cast<const int32_t*>(block_table), context_lens, B, S, Hq, kv_head_num, D, FFKV_BLOCK_SIZE,
+        block_table ? max_context_blocks : 0, block_table ? static_cast<int>(k.shape()[0]) : 0, 0, 0.0f, ws, have,
+        t_stream);
     report(rc, "attention (prefill) failed");
 }
 

@@ -52,6 +52,8 @@
 // zero V rows (their probabilities are exactly zero) and no lane reads outside the cache.
 #include "mfma_common.h"
 
+#include <algorithm>
+
 namespace ffkv
 {
 
@@ -118,6 +120,9 @@ constexpr int kXcds = 8;  // MI355X: workgroups are dealt to 8 XCDs (separate L2
 #ifndef FFKV_PREFILL_V16
 #define FFKV_PREFILL_V16 1  // PV products in f16 for 8-bit caches whose score products are bf16
 #endif
+
+constexpr int kPrefillSplitMin = 4;   // fewest steps of a piece of a split prefill
+constexpr int kPrefillSplitMax = 64;  // most pieces of a row block
 
 #define FFKV_LDS __attribute__((address_space(3)))
 
@@ -254,6 +259,33 @@ __device__ __forceinline__ void wait_vm()
     __builtin_amdgcn_s_waitcnt(VM | (0x7 << 4) | (0xF << 8));  // vmcnt(VM), expcnt and lgkmcnt not waited on
 }
 
+// Pieces that a row block of `steps` steps is split into (a.n_split > 1), the same in every workgroup of the call:
+// as many as keep a piece at kPrefillSplitMin steps or more and all pieces of the call together at about split_slots
+// (the workgroups resident at once).  The call's steps are summed over its rows at the middle of their chunks.
+template <int KP>
+__device__ __forceinline__ int split_pieces(const PrefillArgs& a, int steps, int nrb, int lane)
+{
+    constexpr int KEYS = KP * kBlockSize;
+    if (steps < a.split_from) return 1;
+    int64_t total = 0;
+    for (int b0 = 0; b0 < a.batch; b0 += 64)
+    {
+        int st = 0;
+        if (b0 + lane < a.batch)
+        {
+            int64_t n = (a.paged ? static_cast<int64_t>(a.context_lens[b0 + lane]) : 0) + (a.seq_len + 1) / 2;
+            n = n < 0 ? 0 : (n > a.cap_tokens ? a.cap_tokens : n);
+            st = static_cast<int>((n + KEYS - 1) / KEYS);
+        }
+        total += uniform(wave_sum(st));
+    }
+    total *= static_cast<int64_t>(a.num_kv_heads) * nrb;
+    int64_t len = (total + a.split_slots - 1) / a.split_slots;
+    len = len < kPrefillSplitMin ? kPrefillSplitMin : len;
+    const int np = static_cast<int>((steps + len - 1) / len);
+    return np < 1 ? 1 : (np > a.n_split ? a.n_split : np);
+}
+
 }  // namespace
 
 // PFX = false: prefill (the contract above).  PFX = true: split-K partials of decode queries over a prefix of
@@ -354,7 +386,11 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
     const int Hkv = a.num_kv_heads;
     const int R = PFX ? a.batch * G : S * G;  // query rows of a group: (token, head) or (row, head) pairs
     const int nrb = (R + kDmaRows - 1) / kDmaRows;
-    const int groups = PFX ? Hkv * a.pfx_chunks : a.batch * Hkv;
+    // a prefill split over its keys deals piece p of every group after piece p - 1 of all of them, so that the pieces
+    // of one group spread over the XCDs where the groups are fewer
+    const int groups0 = PFX ? Hkv * a.pfx_chunks : a.batch * Hkv;
+    const int nsp = PFX || a.n_split < 1 ? 1 : a.n_split;
+    const int groups = groups0 * nsp;
 #if FFKV_PREFILL_XCD
     const int wg = wg_index;
     const int xcd = wg % kXcds;
@@ -367,7 +403,7 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
         // The XCD's groups by decreasing cached length (ties by index): lane j ranks group j * kXcds + xcd, and
         // the workgroup takes the group ranked k_in_xcd / nrb.  Absent groups (past `groups`) rank last.
         const int gl = lane * kXcds + xcd;
-        const int wl = lane < g8 && gl < groups ? a.context_lens[gl / a.num_kv_heads] : -2147483647 - 1;
+        const int wl = lane < g8 && gl < groups ? a.context_lens[gl % groups0 / Hkv] : -2147483647 - 1;
         int       rank = 0;
         for (int m = 0; m < g8; ++m)
         {
@@ -382,8 +418,10 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
     const int grp = wg_index / nrb;
     const int rb = wg_index % nrb;
 #endif
-    const int b = PFX ? 0 : grp / Hkv;                 // prefill: the workgroup's row
-    const int kvh = PFX ? grp / a.pfx_chunks : grp % Hkv;
+    const int piece = PFX ? 0 : grp / groups0;
+    const int grp0 = grp - piece * groups0;
+    const int b = PFX ? 0 : grp0 / Hkv;                 // prefill: the workgroup's row
+    const int kvh = PFX ? grp / a.pfx_chunks : grp0 % Hkv;
     const int chunk = PFX ? grp % a.pfx_chunks : 0;  // prefix: pages chunk*pfx_chunk_pages ..
     const int row0 = rb * kDmaRows;
     if (row0 >= R) return;  // uniform over the workgroup
@@ -443,6 +481,21 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
         kw = kw > L ? L : (kw < 0 ? 0 : kw);
         pg_lo = 0;
         pg_hi = static_cast<int>((kw + kBlockSize - 1) / kBlockSize);
+    }
+    int64_t part = -1;  // slot of this piece's partials, or -1: the workgroup has all the keys and writes the output
+    if (!PFX && nsp > 1)
+    {
+        const int np = split_pieces<KP>(a, (pg_hi + KP - 1) / KP, nrb, lane);
+        if (piece >= np) return;  // uniform over the workgroup
+        const int64_t blk = static_cast<int64_t>(grp0) * nrb + rb;
+        if (piece == 0 && tid == 0) a.ws_pieces[blk] = np;
+        if (np > 1)
+        {
+            const int st = (pg_hi + KP - 1) / KP;
+            part = blk * nsp + piece;
+            pg_lo = static_cast<int>(static_cast<int64_t>(st) * piece / np) * KP;
+            pg_hi = min(pg_hi, static_cast<int>(static_cast<int64_t>(st) * (piece + 1) / np) * KP);
+        }
     }
     // uniform values computed through divisions: keep them scalar so the loop's branches stay scalar
     pg_lo = __builtin_amdgcn_readfirstlane(pg_lo);
@@ -1229,6 +1282,24 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
                 }
             }
         }
+        else if (part >= 0)
+        {
+            // partial of the row block's piece: the accumulators as the lanes hold them (whole 1 KiB stores), one
+            // (max in the log2 domain, denominator) per query row
+            if (col_ok[gi])
+            {
+                const int rg = RG * wave + gi;
+                f32x4*    dst = reinterpret_cast<f32x4*>(a.ws_acc) + (part * (kDmaRows / 16) + rg) * NT * 64 + lane;
+#pragma unroll
+                for (int n = 0; n < NT; ++n) dst[n * 64] = acc[gi][n] * v_head_scale;
+                if (g == 0)
+                {
+                    const float shift = CT == I8 && s_vover != 0 ? kRerunShift : 0.0f;
+                    const float m = m_run[gi] == kNegInf ? kNegInf : m_run[gi] * c_log2 - shift;
+                    reinterpret_cast<float2*>(a.ws_ml)[part * kDmaRows + 16 * rg + c] = float2{m, l_tot};
+                }
+            }
+        }
         else if (col_ok[gi])
         {
             const float  inv = l_tot > 0.0f ? v_head_scale / l_tot : 0.0f;
@@ -1255,15 +1326,141 @@ void paged_prefill_dma(PrefillArgs a)
 
 #ifndef FFKV_DEVICE_BODIES_ONLY
 
+// Merge of a prefill split over its keys: thread k of row block blockIdx.y holds lane k % 64 of accumulator k / 64
+// (row group, output tile) of each of the block's pieces, as the pieces' waves wrote them, and writes its four output
+// dims.  A piece that saw no key of the row weighs nothing (its accumulators still enter with weight 0, so that a NaN
+// the row would have met in one pass is met here too).
+template <int QT, int D>
+__global__ __launch_bounds__(256) void paged_prefill_merge(PrefillArgs a)
+{
+    constexpr int NT = D / 16;
+    constexpr int MF = 8;  // pieces whose loads go out together
+    const int     blk = static_cast<int>(blockIdx.y);
+    const int     np = a.ws_pieces[blk];
+    if (np <= 1) return;
+    const int G = a.group, S = a.seq_len, Hkv = a.num_kv_heads;
+    const int nrb = (S * G + kDmaRows - 1) / kDmaRows;
+    const int grp = blk / nrb;
+    const int k = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+    const int lane = k & 63;
+    const int n = (k >> 6) % NT;
+    const int rg = (k >> 6) / NT;
+    const int row = 16 * rg + (lane & 15);
+    const int r = (blk - grp * nrb) * kDmaRows + row;
+    if (r >= S * G) return;
+    const int64_t p0 = static_cast<int64_t>(blk) * a.n_split;
+    const float2* ml = reinterpret_cast<const float2*>(a.ws_ml) + p0 * kDmaRows + row;
+    const f32x4*  xs = reinterpret_cast<const f32x4*>(a.ws_acc) + (p0 * (kDmaRows / 16) + rg) * NT * 64 + n * 64 + lane;
+    float         m = kNegInf, l = 0.0f;
+    f32x4         o = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i0 = 0; i0 < np; i0 += MF)
+    {
+        float2 t[MF];
+        f32x4  x[MF];
+        float  mn = m;
+#pragma unroll
+        for (int f = 0; f < MF; ++f)
+        {
+            t[f] = float2{kNegInf, 0.0f};
+            x[f] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (i0 + f < np)
+            {
+                t[f] = ml[static_cast<int64_t>(i0 + f) * kDmaRows];
+                x[f] = xs[static_cast<int64_t>(i0 + f) * (kDmaRows / 16) * NT * 64];
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < MF; ++f) mn = fmaxf(mn, t[f].x);
+        const float ref = mn == kNegInf ? 0.0f : mn;  // no key so far: every weight is 2^-inf = 0
+        const float wa = __builtin_amdgcn_exp2f(m - ref);
+        l *= wa;
+        o *= wa;
+#pragma unroll
+        for (int f = 0; f < MF; ++f)
+        {
+            const float w = __builtin_amdgcn_exp2f(t[f].x - ref);
+            l += t[f].y * w;
+            o += x[f] * w;
+        }
+        m = mn;
+    }
+    const int    h = grp % Hkv * G + r % G;
+    const size_t ob = ((static_cast<size_t>(grp / Hkv) * S + r / G) * a.num_heads + h) * D + 16 * n + 4 * (lane >> 4);
+    store_out4<QT>(a.out, ob, l > 0.0f ? o * (1.0f / l) : f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+}
+
 namespace
 {
+
+// Kernel and workgroup size of a prefill's main launch, for its occupancy.
+struct PrefillKernel
+{
+    const void* fn;
+    int         threads;
+    int         keys;  // keys per step
+};
+
+template <int CT, int QT>
+PrefillKernel prefill_kernel_d(int head_dim)
+{
+    auto k = []<int D, int RG>()
+    {
+        return PrefillKernel{reinterpret_cast<const void*>(paged_prefill_dma<QT, D, CT, false, RG>), 512 / RG,
+                             DmaCfg<D, kElemBytes<CT>, CT == I8, 8 / RG, false>::KP * kBlockSize};
+    };
+    if (head_dim == 64) return k.template operator()<64, FFKV_PREFILL_RG>();
+    if (head_dim == 128) return k.template operator()<128, FFKV_PREFILL_RG>();
+    return k.template operator()<256, FFKV_PREFILL_RG256>();
+}
+
+template <int CT>
+PrefillKernel prefill_kernel_q(const PrefillArgs& a)
+{
+    if (a.qo_dtype == F32) return prefill_kernel_d<CT, F32>(a.head_dim);
+    if (a.qo_dtype == F16) return prefill_kernel_d<CT, F16>(a.head_dim);
+    return prefill_kernel_d<CT, BF16>(a.head_dim);
+}
+
+PrefillKernel prefill_kernel(const PrefillArgs& a)
+{
+    if (a.cache_dtype == F16) return prefill_kernel_q<F16>(a);
+    if (a.cache_dtype == BF16) return prefill_kernel_q<BF16>(a);
+    if (a.cache_dtype == I8) return prefill_kernel_q<I8>(a);
+    return prefill_kernel_q<FP8>(a);
+}
+
+int64_t prefill_row_blocks(const PrefillArgs& a)
+{
+    return static_cast<int64_t>(a.batch) * a.num_kv_heads *
+           ((static_cast<int64_t>(a.seq_len) * a.group + kDmaRows - 1) / kDmaRows);
+}
+
+template <int QT>
+hipError_t launch_prefill_merge_q(const PrefillArgs& a, hipStream_t stream)
+{
+    const unsigned nb = static_cast<unsigned>(prefill_row_blocks(a));
+    const dim3     grid(static_cast<unsigned>(kDmaRows * a.head_dim / 4 / 256), nb);
+    switch (a.head_dim)
+    {
+        case 64:
+            hipLaunchKernelGGL((paged_prefill_merge<QT, 64>), grid, dim3(256), 0, stream, a);
+            break;
+        case 128:
+            hipLaunchKernelGGL((paged_prefill_merge<QT, 128>), grid, dim3(256), 0, stream, a);
+            break;
+        default:
+            hipLaunchKernelGGL((paged_prefill_merge<QT, 256>), grid, dim3(256), 0, stream, a);
+            break;
+    }
+    return hipGetLastError();
+}
 
 template <int CT, int QT, bool PFX>
 hipError_t launch_pfd_d(const PrefillArgs& a, hipStream_t stream)
 {
     const int64_t rows = PFX ? static_cast<int64_t>(a.batch) * a.group : static_cast<int64_t>(a.seq_len) * a.group;
     const int64_t groups = PFX ? static_cast<int64_t>(a.num_kv_heads) * a.pfx_chunks
-                               : static_cast<int64_t>(a.batch) * a.num_kv_heads;
+                               : static_cast<int64_t>(a.batch) * a.num_kv_heads * (a.n_split > 1 ? a.n_split : 1);
     const int64_t nrb = (rows + kDmaRows - 1) / kDmaRows;
 #if FFKV_PREFILL_XCD
     const int64_t wgs = (groups + kXcds - 1) / kXcds * kXcds * nrb;
@@ -1329,7 +1526,54 @@ hipError_t launch_pfd(const PrefillArgs& a, hipStream_t stream)
 
 }  // namespace
 
-hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream) { return launch_pfd<false>(a, stream); }
+// A prefill with fewer blocks of 128 query rows than workgroups fit the chip at once leaves it partly idle, and its
+// duration is the longest block's: one request's 256 tokens over 7.9k cached ones at 32 / 8 heads are 64 blocks of 132
+// steps on 64 of 256 CUs.  With k times the blocks resident at once, each block is split into k pieces (223 -> 62 us for
+// that call, of which 7.5 us are the merge; 4 pieces took 75 us, 16 took 61, 32 took 69).  A piece's partials (64 KiB at
+// head_dim 128) and the merge cost about as much as 5 steps, so short blocks stay whole: at 4 and more pieces, 16 steps
+// gain (40 -> 28 us), 8 lose (a 500-token prompt: 19.7 -> 23.4 us); at two pieces, which only put a second workgroup on
+// each CU, 31 steps gain (67.8 -> 62.4 us) and 16 lose (30.7 -> 34.7 us).
+void prefill_plan(PrefillArgs& a)
+{
+    a.n_split = 1;
+    a.split_slots = 0;
+    a.split_from = 0;
+    const int64_t       blocks = prefill_row_blocks(a);
+    const PrefillKernel k = prefill_kernel(a);
+    const int           slots = decode_mfma_items(k.fn, k.threads, 1);
+    if (blocks <= 0 || 2 * blocks > slots) return;
+    int64_t       n = slots / blocks;
+    const int     from = n >= 4 ? 12 : (n == 3 ? 16 : 24);
+    const int64_t steps = (static_cast<int64_t>(a.cap_tokens) + k.keys - 1) / k.keys;  // most steps of a block
+    if (steps < from) return;
+    n = std::min(std::min(n, steps / kPrefillSplitMin), static_cast<int64_t>(kPrefillSplitMax));
+    a.n_split = static_cast<int>(n);
+    a.split_slots = slots;
+    a.split_from = from;
+}
+
+PrefillSplitLayout prefill_split_layout(const PrefillArgs& a)
+{
+    if (a.n_split <= 1) return PrefillSplitLayout{};
+    auto               up = [](int64_t x) { return (x + 255) / 256 * 256; };
+    const int64_t      blocks = prefill_row_blocks(a);
+    const int64_t      parts = blocks * a.n_split * kDmaRows;  // query rows of all partials
+    PrefillSplitLayout l{};
+    l.pieces = 0;
+    l.ml = up(blocks * 4);
+    l.acc = l.ml + up(parts * 8);
+    l.total = l.acc + parts * a.head_dim * 4;
+    return l;
+}
+
+hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream)
+{
+    const hipError_t e = launch_pfd<false>(a, stream);
+    if (e != hipSuccess || a.n_split <= 1) return e;
+    if (a.qo_dtype == F32) return launch_prefill_merge_q<F32>(a, stream);
+    if (a.qo_dtype == F16) return launch_prefill_merge_q<F16>(a, stream);
+    return launch_prefill_merge_q<BF16>(a, stream);
+}
 
 hipError_t launch_prefix_partials(const PrefillArgs& a, hipStream_t stream) { return launch_pfd<true>(a, stream); }
 

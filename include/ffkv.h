@@ -219,6 +219,25 @@ FFKV_API int ffkv_paged_prefill(const void* q, void* out, int qo_dtype, const vo
                                 float scale, void* stream);
 
 /*
+ * ffkv_paged_prefill with scratch: a call with too few blocks of 128 query rows to fill the GPU (one request's chunk
+ * over a long context, a short prompt) splits their keys into pieces that run side by side, whose partial results
+ * live in `workspace` (ffkv_prefill_workspace_bytes; 16-byte aligned, any initial contents), and merges them.  Results
+ * equal ffkv_paged_prefill's up to floating-point summation order.  ffkv_prefill_workspace_bytes is 0 where the call
+ * would not be split; with workspace NULL, or fewer bytes than that, the call runs unsplit, as ffkv_paged_prefill.
+ * Calls sharing one workspace must not overlap in time.  paged: whether the call has a block table.
+ */
+FFKV_API size_t ffkv_prefill_workspace_bytes(int qo_dtype, int cache_dtype, int batch, int seq_len, int num_heads,
+                                             int num_kv_heads, int head_dim, int paged, int max_blocks,
+                                             int max_context_len);
+
+FFKV_API int ffkv_paged_prefill_ws(const void* q, void* out, int qo_dtype, const void* k_cache, const void* v_cache,
+                                   int cache_dtype, const float* k_scale, const float* v_scale,
+                                   const int32_t* block_table, const int32_t* context_lens, int batch, int seq_len,
+                                   int num_heads, int num_kv_heads, int head_dim, int block_size, int max_blocks,
+                                   int num_blocks, int max_context_len, float scale, void* workspace,
+                                   size_t workspace_bytes, void* stream);
+
+/*
  * Rotary position embedding of q and k in place.  Replaces `firefly::kernels::apply_rope(q, k, head_dim, seq_len,
  * theta, context_lens)` (include/firefly/kernels.h:68, src/kernels/rope.cu:22-137, called at
  * src/model/qwen_model.cu:136).  q [batch, seq_len, num_heads, head_dim] and k [batch, seq_len, num_kv_heads,

@@ -1,0 +1,144 @@
+"""Prefill split over its keys (few blocks of 128 query rows over many keys) against the CPU closed form and against
+the unsplit call.
+
+Bar against the closed form as in test_gpu_prefill.py.  Split and unsplit differ by the order of fp32 sums and the
+reference maxima of P's rounding to 11 bits: both lie within the bar, so their difference is held to the sum of two.
+Each case says whether the library splits it (``ffkv_prefill_workspace_bytes``), at the edges of the rule: 12 steps of
+64 keys at four pieces and more, 24 at two.
+"""
+
+import numpy as np
+import pytest
+
+import cases
+import gpu_util as gu
+import oracle as O
+from test_gpu_prefill import _case, _check, half_ulp
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(ff, dev, c, qn, contiguous):
+    """(split output, unsplit output, closed form, split?) of the case's chunk."""
+    import torch
+
+    q = gu.to_dev(qn, c.act, dev)
+    B, S, Hq, D = q.shape
+    if contiguous:
+        k, v = gu.to_dev(c.k_new, c.act, dev), gu.to_dev(c.v_new, c.act, dev)
+        ks = vs = bt = cx = None
+        ref = O.paged_prefill_f64(qn, c.act, c.k_new, c.v_new, c.act, None, None)
+    else:
+        k, v = gu.to_dev(c.k_pool, c.kv, dev), gu.to_dev(c.v_pool, c.kv, dev)
+        ks = None if c.k_scale is None else torch.from_numpy(c.k_scale.copy()).to(dev)
+        vs = None if c.v_scale is None else torch.from_numpy(c.v_scale.copy()).to(dev)
+        bt, cx = torch.from_numpy(c.block_table).to(dev), torch.from_numpy(c.ctx).to(dev)
+        ff.append_kv_cache(gu.to_dev(c.k_new, c.act, dev), gu.to_dev(c.v_new, c.act, dev), k, v, bt, cx, ks, vs)
+        rk, rv = c.k_pool.copy(), c.v_pool.copy()
+        rks = None if c.k_scale is None else c.k_scale.copy()
+        rvs = None if c.v_scale is None else c.v_scale.copy()
+        O.append(c.k_new, c.v_new, c.act, rk, rv, c.kv, c.block_table, c.ctx, rks, rvs)
+        ref = O.paged_prefill_f64(qn, c.act, rk, rv, c.kv, c.block_table, c.ctx, rks, rvs)
+    mb = 0 if contiguous else c.max_blocks
+    qt, ct = ff.torch_dtype_code(q), ff.torch_dtype_code(k)
+    need = ff.lib.ffkv_prefill_workspace_bytes(qt, ct, B, S, Hq, c.Hkv, D, int(not contiguous), mb, 0)
+    split = ff.paged_prefill(q, k, v, bt, cx, k_scale=ks, v_scale=vs)
+    whole = torch.full_like(split, float("nan"))
+    ff.check(ff.lib.ffkv_paged_prefill(ff._ptr(q), ff._ptr(whole), qt, ff._ptr(k), ff._ptr(v), ct, ff._ptr(ks),
+                                       ff._ptr(vs), ff._ptr(bt), ff._ptr(cx), B, S, Hq, c.Hkv, D, 16, mb,
+                                       0 if contiguous else c.num_blocks, 0, 0.0, ff._stream(None)))
+    torch.cuda.synchronize()
+    f = lambda t: t.float().cpu().numpy().reshape(ref.shape)
+    return f(split), f(whole), ref, need > 0
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,ctx,S,act,kv,splits", [
+    (1, 32, 8, 128, [1500], 33, "bf16", "bf16", True),    # a remainder of a row block, pieces of 4 and 5 steps
+    (1, 32, 8, 128, [703], 1, "bf16", "bf16", False),     # 11 steps: whole
+    (1, 32, 8, 128, [704], 1, "bf16", "bf16", True),      # 12 steps, the last of one key
+    (1, 2, 2, 128, [4000], 128, "f16", "f16", True),      # two groups over eight XCDs, one full row block each
+    (2, 32, 8, 128, [0, 1200], 130, "f16", "f16", True),  # one row too short to split beside one that is split
+    (3, 10, 2, 64, [900, 1111, 17], 50, "bf16", "bf16", True),
+    (1, 8, 4, 256, [1000], 20, "bf16", "bf16", True),
+    (1, 28, 4, 128, [1000], 70, "f32", "bf16", True),
+    (2, 16, 4, 128, [1000, 850], 40, "bf16", "i8", True),
+    (2, 16, 4, 128, [1000, 850], 40, "bf16", "fp8", True),
+    (1, 8, 4, 64, [2100], 30, "f16", "i8", True),
+])
+def test_split_prefill(ff, gpu, B, Hq, Hkv, D, ctx, S, act, kv, splits):
+    c, qn = _case(900 + S + D, B, Hq, Hkv, D, ctx, S, act=act, kv=kv)
+    got, whole, ref, split = _both(ff, gpu, c, qn, False)
+    assert split == splits
+    tol = 2e-2 if kv in ("i8", "fp8") else 2e-3
+    _check(got, ref, c.act, tol)
+    d = np.abs(got - whole) - 2 * half_ulp(np.maximum(np.abs(got), np.abs(whole)), c.act)
+    assert float(d.max()) <= 2 * tol
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,splits", [(770, 4, 2, True), (700, 4, 2, False)])
+def test_split_prompt(ff, gpu, S, Hq, Hkv, splits):
+    """A whole prompt (contiguous K/V): its late row blocks are split, the early ones are not."""
+    c, qn = _case(950 + S, 1, Hq, Hkv, 128, [0], S, act="f16")
+    got, whole, ref, split = _both(ff, gpu, c, qn, True)
+    assert split == splits
+    _check(got, ref, c.act, 2e-3)
+
+
+def test_split_prefill_reuses_scratch(ff, gpu):
+    """Calls of different sizes in a row, their scratch handed on by the allocator with the former call's contents."""
+    import torch
+
+    for seed, ctx, S in ((1, [3000], 8), (2, [900, 1400], 100), (3, [1300], 3)):
+        c, qn = _case(960 + seed, len(ctx), 8, 2, 128, ctx, S)
+        got, _, ref, split = _both(ff, gpu, c, qn, False)
+        assert split
+        _check(got, ref, c.act, 2e-3)
+    junk = torch.full((64 << 20,), 255, dtype=torch.uint8, device=gpu)
+    del junk
+    got, _, ref, _ = _both(ff, gpu, c, qn, False)
+    _check(got, ref, c.act, 2e-3)
+
+
+def test_split_prefill_masks(ff, gpu):
+    """Absent pages across pieces (a whole piece among them) and a value that only some queries may see."""
+    c, qn = _case(970, 1, 8, 2, 128, [1500], 20)
+    c.block_table[0, 8:30] = -1
+    c.block_table[0, 60] = c.num_blocks + 5
+    got, _, ref, split = _both(ff, gpu, c, qn, False)
+    assert split
+    _check(got, ref, c.act, 2e-3)
+
+
+def test_split_prefill_large_v(ff, gpu):
+    """V beyond f16 in one piece only: that piece's rerun on bf16 products, the others' f16 tiles."""
+    c, qn = _case(980, 1, 8, 2, 128, [1500], 20)
+    page = int(c.block_table[0, 3])
+    v = cases.decode(c.v_pool, c.kv)
+    v[page, 5] *= 1e5
+    c.v_pool = cases.encode(v, c.kv)
+    got, _, ref, split = _both(ff, gpu, c, qn, False)
+    assert split
+    err = np.abs(got - ref)
+    assert float((err / np.maximum(np.abs(ref), 1.0)).max()) < 1e-2
+
+
+def test_unsplit_under_capture(ff, gpu):
+    """A captured call allocates nothing: it runs unsplit, and its replays give the eager call's results."""
+    import torch
+
+    c, qn = _case(990, 1, 8, 2, 128, [1500], 20)
+    q = gu.to_dev(qn, c.act, gpu)
+    kp, vp = gu.to_dev(c.k_pool, c.kv, gpu), gu.to_dev(c.v_pool, c.kv, gpu)
+    bt, cx = torch.from_numpy(c.block_table).to(gpu), torch.from_numpy(c.ctx).to(gpu)
+    eager = ff.paged_prefill(q, kp, vp, bt, cx).clone()
+    out = torch.empty_like(eager)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ff.paged_prefill(q, kp, vp, bt, cx, out=out)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert float((out.float() - eager.float()).abs().max()) <= 4e-3
+        ff.paged_prefill(q, kp, vp, bt, cx)
