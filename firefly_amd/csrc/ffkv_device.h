@@ -415,6 +415,23 @@ __device__ __forceinline__ void load_act8(const void* base, int dt, size_t i, fl
     }
 }
 
+// 4 elements at element index i (a multiple of 4).
+__device__ __forceinline__ void load_act4(const void* base, int dt, size_t i, float* x)
+{
+    if (dt == F32)
+    {
+        const float4 v = *reinterpret_cast<const float4*>(static_cast<const float*>(base) + i);
+        x[0] = v.x, x[1] = v.y, x[2] = v.z, x[3] = v.w;
+    }
+    else
+    {
+        const uint2 v = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(base) + i);
+        const uint32_t h[4] = {v.x & 0xffffu, v.x >> 16, v.y & 0xffffu, v.y >> 16};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = dt == F16 ? f16_to_f32(h[k]) : bf16_to_f32(h[k]);
+    }
+}
+
 __device__ __forceinline__ void store_act1(void* base, int dt, size_t i, float x)
 {
     if (dt == F32)

@@ -26,15 +26,48 @@ namespace
 {
 
 #ifndef FFKV_GENERIC_U16
-#define FFKV_GENERIC_U16 4
+#define FFKV_GENERIC_U16 4  // token groups per loop trip: other caches
 #endif
 #ifndef FFKV_GENERIC_U32
-#define FFKV_GENERIC_U32 2
+#define FFKV_GENERIC_U32 2  // token groups per loop trip: fp32 caches (a raw row takes twice the registers)
 #endif
 
 constexpr float kNegBig = -1e30f;  // finite "minus infinity" seed, as in attention.cu:323
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
+
+// Dims held by a lane of a D-dim row, the same for q, K, V and the output: 8 consecutive ones (16 bytes of a 16-bit
+// cache).  A lane's 8 fp32 values are two 16-byte loads, so they come from the row's two halves, four from each:
+// either load then covers whole lines of consecutive lanes, where 8 consecutive dims would have both loads touch
+// every line.
+template <int CT>
+__device__ __forceinline__ int lane_dim(int D, int lane, int i)
+{
+    return CT == F32 ? (i >> 2) * (D >> 1) + 4 * lane + (i & 3) : 8 * lane + i;
+}
+
+template <int CT, bool NT>
+__device__ __forceinline__ void load_row8(const void* base, size_t row, int D, int lane, Raw8& r)
+{
+    if constexpr (CT == F32)
+    {
+        const float* p = static_cast<const float*>(base) + row * D;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+        {
+            const u32x4* s = reinterpret_cast<const u32x4*>(p + lane_dim<CT>(D, lane, 4 * h));
+            const u32x4  w = NT ? __builtin_nontemporal_load(s) : *s;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r.w[4 * h + i] = w[i];
+        }
+    }
+    else
+    {
+        load_raw8<CT>(base, row * D + lane * 8, r);
+    }
+}
 
 __device__ __forceinline__ int row_tokens(const DecodeArgs& a, int b)
 {
@@ -77,7 +110,16 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
     for (int g = 0; g < GP; ++g)
     {
         if (g < G && act)
-            load_act8(a.q, a.qo_dtype, (static_cast<size_t>(b) * a.num_heads + kvh * G + g) * D + lane * 8, q[g]);
+        {
+            const size_t qb = (static_cast<size_t>(b) * a.num_heads + kvh * G + g) * D;
+            if constexpr (CT == F32)
+            {
+                load_act4(a.q, a.qo_dtype, qb + lane_dim<CT>(D, lane, 0), q[g]);
+                load_act4(a.q, a.qo_dtype, qb + lane_dim<CT>(D, lane, 4), q[g] + 4);
+            }
+            else
+                load_act8(a.q, a.qo_dtype, qb + lane * 8, q[g]);
+        }
         else
 #pragma unroll
             for (int i = 0; i < 8; ++i) q[g][i] = 0.0f;
@@ -93,113 +135,135 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
         for (int i = 0; i < 8; ++i) acc[g][i] = 0.0f;
     }
 
-    // U consecutive token groups per loop trip: their table entries, then all their K / V loads, go out before
-    // any of them is used, so U times the bytes of one group are in flight per wave (fewer for fp32 caches, whose
-    // raw rows take twice the registers, and none extra for the 16-head groups, which already fill them).
-    constexpr int  U = GP >= 16 ? 1 : (Storage<CT>::bytes == 4 ? FFKV_GENERIC_U32 : FFKV_GENERIC_U16);
-    // The table entries of the next trip are requested while this trip's tokens are computed.
+    // fp32 pages are read past the caches, unless a neighbouring row holds the chunk's first page too (a shared
+    // prefix, which the rows' workgroups then read from the caches).  32 rows of 512 to 4096 tokens at 32/8 heads take
+    // 128 us per call with plain loads and 114 (5.3 TB/s) with these, 120 rows over a 2048-token prefix 203 us with
+    // plain loads and 275 with these.  (Four token groups per trip gain another 1 % on the former and cost the latter
+    // 10 %: fewer waves fit.)
     const int32_t* table = a.block_table + static_cast<int64_t>(b) * a.max_blocks;
-    auto load_phys = [&](int base, int (&ph)[U])
+    bool           once = CT == F32;
+    if (CT == F32 && begin < end)
     {
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-        {
-            const int j = base + u * TPI + slot;
-            ph[u] = j < end ? table[j >> 4] : -1;
-        }
-    };
-    int phys[U];
-    load_phys(begin, phys);
-    for (int base = begin; base < end; base += U * TPI)
+        const int own = table[begin >> 4];
+        for (int o = -1; o <= 1; o += 2)
+            if (b + o >= 0 && b + o < a.batch && table[(begin >> 4) + static_cast<int64_t>(o) * a.max_blocks] == own)
+                once = false;
+        once = __builtin_amdgcn_readfirstlane(once);
+    }
+
+    // U consecutive token groups per loop trip: their table entries, then all their K / V loads, go out before
+    // any of them is used, so U times the bytes of one group are in flight per wave (none extra for the 16-head
+    // groups, which already fill the registers).  The table entries of the next trip are requested while this trip's
+    // tokens are computed.
+    auto stream = [&]<int U, bool NT>()
     {
-        bool   valid[U];
-        size_t row[U];
-        float  ks[U], vs[U];  // int8: the tokens' scales
-#pragma unroll
-        for (int u = 0; u < U; ++u)
+        auto load_phys = [&](int base, int (&ph)[U])
         {
-            const int j = base + u * TPI + slot;
-            valid[u] = j < end && phys[u] >= 0 && phys[u] < a.num_blocks;
-            row[u] = (static_cast<size_t>(valid[u] ? phys[u] : 0) * kBlockSize + (j & 15)) * a.num_kv_heads + kvh;
-        }
-        Raw8 kr[U], vr[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-        {
-            ks[u] = vs[u] = 1.0f;
-            if (valid[u] && act)
+            for (int u = 0; u < U; ++u)
             {
-                load_raw8<CT>(a.k_cache, row[u] * D + lane * 8, kr[u]);
-                load_raw8<CT>(a.v_cache, row[u] * D + lane * 8, vr[u]);
-                if constexpr (CT == I8)
+                const int j = base + u * TPI + slot;
+                ph[u] = j < end ? table[j >> 4] : -1;
+            }
+        };
+        int phys[U];
+        load_phys(begin, phys);
+        for (int base = begin; base < end; base += U * TPI)
+        {
+            bool   valid[U];
+            size_t row[U];
+            float  ks[U], vs[U];  // int8: the tokens' scales
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+            {
+                const int j = base + u * TPI + slot;
+                valid[u] = j < end && phys[u] >= 0 && phys[u] < a.num_blocks;
+                row[u] = (static_cast<size_t>(valid[u] ? phys[u] : 0) * kBlockSize + (j & 15)) * a.num_kv_heads + kvh;
+            }
+            Raw8 kr[U], vr[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+            {
+                ks[u] = vs[u] = 1.0f;
+                if (valid[u] && act)
                 {
-                    ks[u] = a.k_scale[row[u]];
-                    vs[u] = a.v_scale[row[u]];
+                    load_row8<CT, NT>(a.k_cache, row[u], D, lane, kr[u]);
+                    load_row8<CT, NT>(a.v_cache, row[u], D, lane, vr[u]);
+                    if constexpr (CT == I8)
+                    {
+                        ks[u] = a.k_scale[row[u]];
+                        vs[u] = a.v_scale[row[u]];
+                    }
+                }
+                else
+                {
+                    kr[u] = Raw8{};
+                    vr[u] = Raw8{};
                 }
             }
-            else
+            load_phys(base + U * TPI, phys);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
             {
-                kr[u] = Raw8{};
-                vr[u] = Raw8{};
-            }
-        }
-        load_phys(base + U * TPI, phys);
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-        {
-            float k[8];
-            unpack8<CT>(kr[u], k);
-            if constexpr (CT == I8 || CT == FP8)
-            {
-                const float sk = CT == I8 ? ks[u] : a.k_scale[kvh];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) k[i] *= sk;
-            }
-            float s[GP];
-#pragma unroll
-            for (int g = 0; g < GP; ++g)
-            {
-                float d = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) d = __builtin_fmaf(q[g][i], k[i], d);
-                s[g] = d;
-            }
-            // every lane takes part in the sums (DPP lane steps); a token's lanes are a contiguous, aligned group
-#pragma unroll
-            for (int g = 0; g < GP; ++g) s[g] = group_sum<LPT>(s[g]);
-
-            // Online softmax with a lazy reference: m moves (and l, acc are rescaled) only when a score exceeds it
-            // by more than 8 (log2 units), so p = 2^(s - m) < 2^8 and most tokens only add p and p * v.
-            if (valid[u])
-            {
-                float v[8];  // unpacked only now: fewer registers live across the dot products and sums
-                unpack8<CT>(vr[u], v);
+                float k[8];
+                unpack8<CT>(kr[u], k);
                 if constexpr (CT == I8 || CT == FP8)
                 {
-                    const float sv = CT == I8 ? vs[u] : a.v_scale[kvh];
+                    const float sk = CT == I8 ? ks[u] : a.k_scale[kvh];
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) v[i] *= sv;
+                    for (int i = 0; i < 8; ++i) k[i] *= sk;
                 }
+                float s[GP];
 #pragma unroll
                 for (int g = 0; g < GP; ++g)
                 {
-                    const float sg = s[g] * a.scale_log2;
-                    if (sg > m[g] + 8.0f)
+                    float d = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) d = __builtin_fmaf(q[g][i], k[i], d);
+                    s[g] = d;
+                }
+                // every lane takes part in the sums (DPP lane steps); a token's lanes are a contiguous, aligned group
+#pragma unroll
+                for (int g = 0; g < GP; ++g) s[g] = group_sum<LPT>(s[g]);
+
+                // Online softmax with a lazy reference: m moves (and l, acc are rescaled) only when a score exceeds it
+                // by more than 8 (log2 units), so p = 2^(s - m) < 2^8 and most tokens only add p and p * v.
+                if (valid[u])
+                {
+                    float v[8];  // unpacked only now: fewer registers live across the dot products and sums
+                    unpack8<CT>(vr[u], v);
+                    if constexpr (CT == I8 || CT == FP8)
                     {
-                        const float alpha = fast_exp2(m[g] - sg);  // 0 for the slot's first token
-                        l[g] *= alpha;
+                        const float sv = CT == I8 ? vs[u] : a.v_scale[kvh];
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) acc[g][i] *= alpha;
-                        m[g] = sg;
+                        for (int i = 0; i < 8; ++i) v[i] *= sv;
                     }
-                    const float p = fast_exp2(sg - m[g]);
-                    l[g] += p;
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) acc[g][i] = __builtin_fmaf(p, v[i], acc[g][i]);
+                    for (int g = 0; g < GP; ++g)
+                    {
+                        const float sg = s[g] * a.scale_log2;
+                        if (sg > m[g] + 8.0f)
+                        {
+                            const float alpha = fast_exp2(m[g] - sg);  // 0 for the slot's first token
+                            l[g] *= alpha;
+#pragma unroll
+                            for (int i = 0; i < 8; ++i) acc[g][i] *= alpha;
+                            m[g] = sg;
+                        }
+                        const float p = fast_exp2(sg - m[g]);
+                        l[g] += p;
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) acc[g][i] = __builtin_fmaf(p, v[i], acc[g][i]);
+                    }
                 }
             }
         }
-    }
+    };
+    constexpr int U = GP >= 16 ? 1 : (CT == F32 ? FFKV_GENERIC_U32 : FFKV_GENERIC_U16);
+    if (CT == F32 && once)
+        stream.template operator()<U, CT == F32>();
+    else
+        stream.template operator()<U, false>();
 
     // merge the token slots of this wave (lanes lane, lane+LPT, ... hold the same dims)
 #pragma unroll
@@ -235,7 +299,7 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
                 if (w == 0)
                 {
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) s_acc[g][lane * 8 + i] = acc[g][i];
+                    for (int i = 0; i < 8; ++i) s_acc[g][lane_dim<CT>(D, lane, i)] = acc[g][i];
                     if (lane == 0)
                     {
                         s_m[g] = m[g];
@@ -251,7 +315,10 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
                     const float a2 = fast_exp2(mo - mn);
 #pragma unroll
                     for (int i = 0; i < 8; ++i)
-                        s_acc[g][lane * 8 + i] = acc[g][i] * a1 + s_acc[g][lane * 8 + i] * a2;
+                    {
+                        float& o = s_acc[g][lane_dim<CT>(D, lane, i)];
+                        o = acc[g][i] * a1 + o * a2;
+                    }
                     // all holder lanes read s_m/s_l before lane 0 overwrites them: same wave, lockstep
                     __builtin_amdgcn_wave_barrier();
                     if (lane == 0)
@@ -292,29 +359,58 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
     }
 }
 
-// Combine the chunk partials of rows that needed more than one chunk.  One workgroup per (query head, row).
+// Combine the chunk partials of rows that needed more than one chunk: thread k of row b's workgroups folds dims
+// 4 (k % (D/4)) .. + 3 of head k / (D/4) over the row's chunks, the loads of MF chunks in flight together (one
+// workgroup per head, its threads walking the chunks three times with one load in flight, took 11.6 us on 32 rows of
+// 512 to 4096 tokens; this takes 5.0).
 __global__ __launch_bounds__(256) void paged_decode_merge(DecodeArgs a)
 {
-    const int D = a.head_dim;
-    const int hq = blockIdx.x;
-    const int b = blockIdx.y;
-    const int L = row_tokens(a, b);
-    const int nch = (L + a.chunk - 1) / a.chunk;
-    if (nch <= 1) return;
-
-    const int64_t base = (static_cast<int64_t>(b) * a.num_heads + hq) * a.max_chunks;
-    float         M = kNegBig;
-    for (int c = 0; c < nch; ++c) M = fmaxf(M, a.ws_ml[2 * (base + c)]);
-    float lsum = 0.0f;
-    for (int c = 0; c < nch; ++c) lsum += a.ws_ml[2 * (base + c) + 1] * fast_exp2(a.ws_ml[2 * (base + c)] - M);
-    const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
-    for (int d = threadIdx.x; d < D; d += 256)
+    constexpr int MF = 8;
+    const int     D = a.head_dim;
+    const int     b = blockIdx.x;
+    const int     k = static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x);
+    const int     L = row_tokens(a, b);
+    const int     nch = (L + a.chunk - 1) / a.chunk;
+    if (nch <= 1 || k >= a.num_heads * (D / 4)) return;
+    const int     h = k / (D / 4);
+    const int     d4 = (k - h * (D / 4)) * 4;
+    const int64_t base = (static_cast<int64_t>(b) * a.num_heads + h) * a.max_chunks;
+    float         m = kNegBig, l = 0.0f, o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c0 = 0; c0 < nch; c0 += MF)
     {
-        float o = 0.0f;
-        for (int c = 0; c < nch; ++c)
-            o += a.ws_acc[(base + c) * D + d] * fast_exp2(a.ws_ml[2 * (base + c)] - M);
-        store_act1(a.out, a.qo_dtype, (static_cast<size_t>(b) * a.num_heads + hq) * D + d, o * inv);
+        float2 t[MF];
+        float4 x[MF];
+        float  mn = m;
+#pragma unroll
+        for (int f = 0; f < MF; ++f)
+        {
+            t[f] = make_float2(kNegBig, 0.0f);
+            x[f] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (c0 + f < nch)
+            {
+                t[f] = *reinterpret_cast<const float2*>(a.ws_ml + 2 * (base + c0 + f));
+                x[f] = *reinterpret_cast<const float4*>(a.ws_acc + (base + c0 + f) * D + d4);
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < MF; ++f) mn = fmaxf(mn, t[f].x);
+        const float wa = fast_exp2(m - mn);
+        l *= wa;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] *= wa;
+#pragma unroll
+        for (int f = 0; f < MF; ++f)
+        {
+            const float w = fast_exp2(t[f].x - mn);
+            l += t[f].y * w;
+            o[0] += x[f].x * w, o[1] += x[f].y * w, o[2] += x[f].z * w, o[3] += x[f].w * w;
+        }
+        m = mn;
     }
+    const float  inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const size_t ob = (static_cast<size_t>(b) * a.num_heads + h) * D + d4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) store_act1(a.out, a.qo_dtype, ob + i, o[i] * inv);
 }
 
 namespace
@@ -328,8 +424,10 @@ hipError_t launch3(const DecodeArgs& a, hipStream_t stream)
     hipLaunchKernelGGL((paged_decode_generic<CT, DT, LPT, GP>), grid, dim3(256), 0, stream, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.max_chunks <= 1) return e;
-    hipLaunchKernelGGL(paged_decode_merge, dim3(static_cast<unsigned>(a.num_heads), static_cast<unsigned>(a.batch)),
-                       dim3(a.head_dim < 256 ? a.head_dim : 256), 0, stream, a);
+    hipLaunchKernelGGL(paged_decode_merge,
+                       dim3(static_cast<unsigned>(a.batch),
+                            static_cast<unsigned>((a.num_heads * (a.head_dim / 4) + 255) / 256)),
+                       dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

@@ -1,0 +1,41 @@
+"""Decode over fp32 pages: the lanes' split of a row's dims over its two halves, the loads that go past the caches
+(rows with pages of their own) and those that do not (rows that share their first pages), and the merge of one to many
+chunks (chunks of 256 tokens here, merged eight at a time).  Against the CPU checker, 1e-4 as in test_gpu_parity.py.
+"""
+
+import math
+
+import pytest
+
+import cases
+from test_gpu_parity import _check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,G,ctx", [
+    (128, 4, [0, 255, 256, 2046, 2047, 2048, 2049, 4200]),  # 1, 1, 2, 8, 8, 9, 9 and 17 chunks
+    (64, 1, [300, 2100]),
+    (256, 8, [17, 700, 1025]),
+    (8, 2, [600, 5]),
+    (88, 16, [515, 2300]),
+])
+def test_decode_f32(ff, gpu, D, G, ctx):
+    c = cases.make_case(700 + D + G, len(ctx), 2 * G, 2, D, ctx, act="f32", input_scale=1 / math.sqrt(D))
+    _check(ff, gpu, c, 1e-4)
+
+
+@pytest.mark.parametrize("shared", [1, 20])
+def test_decode_f32_shared_pages(ff, gpu, shared):
+    """Rows that share their first pages with a neighbour, and one in between that ends inside them."""
+    c = cases.make_case(720 + shared, 5, 16, 4, 128, [700, 16 * shared - 1, 900, 333, 16 * shared + 1], act="f32",
+                        input_scale=1 / math.sqrt(128), shared_prefix_blocks=shared)
+    c.ctx[1] = 16 * shared - 2  # its new token stays out of the shared pages' last slot
+    _check(ff, gpu, c, 1e-4)
+
+
+@pytest.mark.parametrize("kv,tol", [("bf16", 2e-3), ("i8", 2e-2)])
+def test_vector_decode_merge(ff, gpu, kv, tol):
+    """The same merge behind the vector kernel's other caches (head_dim 88)."""
+    c = cases.make_case(740, 3, 12, 3, 88, [2047, 90, 3000], act="bf16", kv=kv, input_scale=1 / math.sqrt(88))
+    _check(ff, gpu, c, tol)
