@@ -12,6 +12,11 @@ import ctypes
 import os
 from pathlib import Path
 
+try:
+    from . import _front
+except ImportError as e:
+    raise ImportError("firefly_amd/_front.so is not built; run `python firefly_amd/build.py`") from e
+
 _PKG = Path(__file__).resolve().parent
 LIB_PATH = _PKG / "libffkv.so"
 
@@ -46,9 +51,9 @@ def _load() -> ctypes.CDLL:
     # makes libffkv.so bind to that already-loaded runtime, so there is one runtime per process and torch's
     # device pointers and streams are valid here; loading ours first would put two runtimes in the process.
     try:
-        import torch  # noqa: F401
+        import torch
     except ImportError:
-        pass
+        torch = None
     lib = ctypes.CDLL(str(LIB_PATH), mode=os.RTLD_NOW | ctypes.RTLD_LOCAL)
     vp, i32, f32, sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_size_t
     lib.ffkv_append.restype = i32
@@ -88,10 +93,18 @@ def _load() -> ctypes.CDLL:
     lib.ffkv_last_error.argtypes = []
     lib.ffkv_version.restype = ctypes.c_char_p
     lib.ffkv_version.argtypes = []
+    if torch is not None:
+        _bind(lib, torch)
     return lib
 
 
-lib = _load()
+def _bind(lib, torch) -> None:
+    """Point the native front end (``_front``, csrc/python/front.cpp) at ``lib``'s functions."""
+    names = ("append", "paged_decode", "append_paged_decode", "paged_decode_shared_prefix", "paged_decode_noalloc",
+             "prefill_workspace_bytes", "paged_prefill_ws", "rope", "rope_append")
+    _front.bind(tuple(ctypes.cast(getattr(lib, "ffkv_" + n), ctypes.c_void_p).value for n in names),
+                list(_torch_dtypes(torch).items()), getattr(torch._C, "_cuda_getDevice", None),
+                getattr(torch._C, "_cuda_getCurrentRawStream", None), lambda: torch.cuda.current_stream().cuda_stream)
 
 
 def version() -> str:
@@ -103,10 +116,8 @@ def check(code: int) -> None:
         raise FFKVError(code, lib.ffkv_last_error().decode())
 
 
-def torch_dtype_code(t) -> int:
-    """ffkv dtype code of a torch tensor (uint8 storage is read as OCP fp8 e4m3)."""
-    import torch
-
+def _torch_dtypes(torch) -> dict:
+    """torch dtype -> ffkv dtype code (uint8 storage is read as OCP fp8 e4m3)."""
     table = {
         torch.float32: DTYPE_F32,
         torch.float16: DTYPE_F16,
@@ -117,10 +128,21 @@ def torch_dtype_code(t) -> int:
     fp8 = getattr(torch, "float8_e4m3fn", None)
     if fp8 is not None:
         table[fp8] = DTYPE_FP8_E4M3
+    return table
+
+
+def torch_dtype_code(t) -> int:
+    """ffkv dtype code of a torch tensor (uint8 storage is read as OCP fp8 e4m3)."""
+    import torch
+
     try:
-        return table[t.dtype]
+        return _torch_dtypes(torch)[t.dtype]
     except KeyError as e:
         raise TypeError(f"unsupported dtype {t.dtype}") from e
+
+
+lib = _load()
+os.register_at_fork(after_in_child=_front.forget_stream)
 
 
 def _ptr(t) -> int | None:
@@ -138,75 +160,51 @@ def _stream(stream) -> int | None:
 def append_kv_cache(k, v, k_cache, v_cache, block_table, context_lens=None, k_scale=None, v_scale=None,
                     num_blocks: int | None = None, stream=None) -> None:
     """Append ``k``/``v`` ``[B, S, Hkv, D]`` into pages ``[N, 16, Hkv, D]`` (``ffkv_append``)."""
-    B, S, Hkv, D = k.shape
-    max_blocks = block_table.shape[-1]
-    N = k_cache.shape[0] if num_blocks is None else num_blocks
-    check(lib.ffkv_append(_ptr(k), _ptr(v), torch_dtype_code(k), _ptr(k_cache), _ptr(v_cache),
-                          torch_dtype_code(k_cache), _ptr(k_scale), _ptr(v_scale), _ptr(block_table),
-                          _ptr(context_lens), B, S, Hkv, D, BLOCK_SIZE, max_blocks, N, _stream(stream)))
+    check(_front.append(k, v, k_cache, v_cache, block_table, context_lens, k_scale, v_scale, num_blocks, stream))
 
 
 def paged_prefill(q, k_cache, v_cache, block_table, context_lens, out=None, k_scale=None, v_scale=None,
                   max_context_len: int = 0, scale: float = 0.0, num_blocks: int | None = None, stream=None):
-    """Causal prefill attention (``ffkv_paged_prefill``): ``q`` ``[B, S, Hq, D]`` over the paged cache (queries at
+    """Causal prefill attention (``ffkv_paged_prefill_ws``): ``q`` ``[B, S, Hq, D]`` over the paged cache (queries at
     ``context_lens[b] + t``), or, with ``block_table=None``, over contiguous ``k_cache``/``v_cache``
     ``[B, S, Hkv, D]``.  Returns ``out`` ``[B, S, Hq * D]``."""
-    import torch
-
-    B, S, Hq, D = q.shape
-    Hkv = k_cache.shape[2]
     if out is None:
+        import torch
+
+        B, S, Hq, D = q.shape
         out = torch.empty((B, S, Hq * D), dtype=q.dtype, device=q.device)
-    max_blocks = 0 if block_table is None else block_table.shape[-1]
-    N = (k_cache.shape[0] if num_blocks is None else num_blocks) if block_table is not None else 0
-    qt, ct = torch_dtype_code(q), torch_dtype_code(k_cache)
-    ws, ws_bytes = _prefill_scratch(lib.ffkv_prefill_workspace_bytes(qt, ct, B, S, Hq, Hkv, D, block_table is not None,
-                                                                     max_blocks, max_context_len), q.device, stream)
-    check(lib.ffkv_paged_prefill_ws(_ptr(q), _ptr(out), qt, _ptr(k_cache), _ptr(v_cache), ct, _ptr(k_scale),
-                                    _ptr(v_scale), _ptr(block_table), _ptr(context_lens), B, S, Hq, Hkv, D, BLOCK_SIZE,
-                                    max_blocks, N, max_context_len, float(scale), _ptr(ws), ws_bytes,
-                                    _stream(stream)))
+    check(_front.prefill(q, out, k_cache, v_cache, k_scale, v_scale, block_table, context_lens, max_context_len, scale,
+                         num_blocks, stream, _prefill_scratch))
     return out
 
 
-def _prefill_scratch(n: int, device, stream):
+def _prefill_scratch(n: int, q, stream):
     """Scratch of ``n`` bytes for one call on ``stream`` (None: the current one), from torch's allocator and belonging
     to that stream, so that it can be reused once the call's work on the stream is done.  None while the stream is
     being captured (a capture allocates nothing here; the call then runs unsplit)."""
     import torch
 
-    if n == 0:
-        return None, 0
     if stream is not None:
         if not isinstance(stream, torch.cuda.Stream):
-            stream = torch.cuda.ExternalStream(int(getattr(stream, "cuda_stream", stream)), device=device)
+            stream = torch.cuda.ExternalStream(int(getattr(stream, "cuda_stream", stream)), device=q.device)
         with torch.cuda.stream(stream):
-            return _prefill_scratch(n, device, None)
+            return _prefill_scratch(n, q, None)
     if torch.cuda.is_current_stream_capturing():
-        return None, 0
-    return torch.empty(n, dtype=torch.uint8, device=device), n
+        return None
+    return torch.empty(n, dtype=torch.uint8, device=q.device)
 
 
 def apply_rope(q, k, context_lens=None, theta: float = 1e6, stream=None) -> None:
     """Rotary embedding of ``q`` ``[B, S, Hq, D]`` (or None) and ``k`` ``[B, S, Hkv, D]`` in place
     (``ffkv_rope``; the reference's ``kernels::apply_rope``)."""
-    B, S, Hkv, D = k.shape
-    Hq = 0 if q is None else q.shape[2]
-    check(lib.ffkv_rope(_ptr(q), _ptr(k), torch_dtype_code(k), _ptr(context_lens), B, S, Hq, Hkv, D, float(theta),
-                        _stream(stream)))
+    check(_front.rope(q, k, context_lens, theta, stream))
 
 
 def rope_append_kv_cache(q, k, v, k_cache, v_cache, block_table, context_lens=None, theta: float = 1e6,
                          k_scale=None, v_scale=None, num_blocks: int | None = None, stream=None) -> None:
     """``apply_rope(q, k)`` then ``append_kv_cache(k, v, ...)`` in one kernel (``ffkv_rope_append``)."""
-    B, S, Hkv, D = k.shape
-    Hq = 0 if q is None else q.shape[2]
-    max_blocks = block_table.shape[-1]
-    N = k_cache.shape[0] if num_blocks is None else num_blocks
-    check(lib.ffkv_rope_append(_ptr(q), _ptr(k), _ptr(v), torch_dtype_code(k), _ptr(k_cache), _ptr(v_cache),
-                               torch_dtype_code(k_cache), _ptr(k_scale), _ptr(v_scale), _ptr(block_table),
-                               _ptr(context_lens), B, S, Hq, Hkv, D, BLOCK_SIZE, max_blocks, N, float(theta),
-                               _stream(stream)))
+    check(_front.rope_append(q, k, v, k_cache, v_cache, block_table, context_lens, theta, k_scale, v_scale, num_blocks,
+                             stream))
 
 
 def kv_block_bytes(cache_dtype: int, num_kv_heads: int, head_dim: int) -> int:
@@ -238,26 +236,23 @@ def shared_prefix_workspace(batch: int, num_heads: int, num_kv_heads: int, head_
     return torch.empty(n, dtype=torch.uint8, device=device if device is not None else "cuda")
 
 
+def _decode_out(q, out):
+    """``out``, or a new ``[B, 1, Hq * D]`` like ``q``."""
+    if out is None:
+        import torch
+
+        out = torch.empty((q.shape[0], 1, q.shape[-2] * q.shape[-1]), dtype=q.dtype, device=q.device)
+    return out
+
+
 def paged_attention_shared_prefix(q, k_cache, v_cache, block_table, context_lens, shared_blocks: int, out=None,
                                   k_scale=None, v_scale=None, max_context_len: int = 0, scale: float = 0.0,
                                   workspace=None, num_blocks: int | None = None, stream=None):
     """Decode over rows whose first ``shared_blocks`` block-table entries are the same pages
     (``ffkv_paged_decode_shared_prefix``): the shared pages are attended once for all rows."""
-    import torch
-
-    B = q.shape[0]
-    Hq, D = q.shape[-2], q.shape[-1]
-    Hkv = k_cache.shape[2]
-    if out is None:
-        out = torch.empty((B, 1, Hq * D), dtype=q.dtype, device=q.device)
-    max_blocks = block_table.shape[-1]
-    N = k_cache.shape[0] if num_blocks is None else num_blocks
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    check(lib.ffkv_paged_decode_shared_prefix(_ptr(q), _ptr(out), torch_dtype_code(q), _ptr(k_cache), _ptr(v_cache),
-                                              torch_dtype_code(k_cache), _ptr(k_scale), _ptr(v_scale),
-                                              _ptr(block_table), _ptr(context_lens), B, Hq, Hkv, D, BLOCK_SIZE,
-                                              max_blocks, N, max_context_len, float(scale), int(shared_blocks),
-                                              _ptr(workspace), ws_bytes, _stream(stream)))
+    out = _decode_out(q, out)
+    check(_front.decode_shared(q, out, k_cache, v_cache, k_scale, v_scale, block_table, context_lens, max_context_len,
+                               scale, num_blocks, int(shared_blocks), workspace, stream))
     return out
 
 
@@ -266,21 +261,9 @@ def append_paged_attention(k_new, v_new, q, k_cache, v_cache, block_table, conte
                            num_blocks: int | None = None, stream=None):
     """``append_kv_cache(k_new, v_new, ...)`` (one token per row) then ``paged_attention``, as one call
     (``ffkv_append_paged_decode``; a single launch for 16-bit caches fed in their own dtype)."""
-    import torch
-
-    B = q.shape[0]
-    Hq, D = q.shape[-2], q.shape[-1]
-    Hkv = k_cache.shape[2]
-    if out is None:
-        out = torch.empty((B, 1, Hq * D), dtype=q.dtype, device=q.device)
-    max_blocks = block_table.shape[-1]
-    N = k_cache.shape[0] if num_blocks is None else num_blocks
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    check(lib.ffkv_append_paged_decode(_ptr(k_new), _ptr(v_new), torch_dtype_code(k_new), _ptr(q), _ptr(out),
-                                       torch_dtype_code(q), _ptr(k_cache), _ptr(v_cache), torch_dtype_code(k_cache),
-                                       _ptr(k_scale), _ptr(v_scale), _ptr(block_table), _ptr(context_lens), B, Hq,
-                                       Hkv, D, BLOCK_SIZE, max_blocks, N, max_context_len, float(scale),
-                                       _ptr(workspace), ws_bytes, _stream(stream)))
+    out = _decode_out(q, out)
+    check(_front.append_decode(q, out, k_cache, v_cache, k_scale, v_scale, block_table, context_lens, max_context_len,
+                               scale, num_blocks, k_new, v_new, workspace, stream))
     return out
 
 
@@ -288,15 +271,8 @@ def paged_attention_noalloc(q, k_cache, v_cache, block_table, context_lens, out,
                             max_context_len: int = 0, scale: float = 0.0, num_blocks: int | None = None, stream=None):
     """PagedAttention decode that allocates no device memory (``ffkv_paged_decode_noalloc``): the split-K partials
     use the library's static per-GPU scratch.  ``out`` ``[B, 1, Hq * D]`` is the caller's."""
-    B = q.shape[0]
-    Hq, D = q.shape[-2], q.shape[-1]
-    Hkv = k_cache.shape[2]
-    max_blocks = block_table.shape[-1]
-    N = k_cache.shape[0] if num_blocks is None else num_blocks
-    check(lib.ffkv_paged_decode_noalloc(_ptr(q), _ptr(out), torch_dtype_code(q), _ptr(k_cache), _ptr(v_cache),
-                                        torch_dtype_code(k_cache), _ptr(k_scale), _ptr(v_scale), _ptr(block_table),
-                                        _ptr(context_lens), B, Hq, Hkv, D, BLOCK_SIZE, max_blocks, N,
-                                        max_context_len, float(scale), _stream(stream)))
+    check(_front.decode_noalloc(q, out, k_cache, v_cache, k_scale, v_scale, block_table, context_lens, max_context_len,
+                                scale, num_blocks, stream))
     return out
 
 
@@ -304,18 +280,7 @@ def paged_attention(q, k_cache, v_cache, block_table, context_lens, out=None, k_
                     max_context_len: int = 0, scale: float = 0.0, workspace=None, num_blocks: int | None = None,
                     stream=None):
     """PagedAttention decode (``ffkv_paged_decode``).  ``q`` is ``[B, 1, Hq, D]`` (or ``[B, Hq, D]``)."""
-    import torch
-
-    B = q.shape[0]
-    Hq, D = q.shape[-2], q.shape[-1]
-    Hkv = k_cache.shape[2]
-    if out is None:
-        out = torch.empty((B, 1, Hq * D), dtype=q.dtype, device=q.device)
-    max_blocks = block_table.shape[-1]
-    N = k_cache.shape[0] if num_blocks is None else num_blocks
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    check(lib.ffkv_paged_decode(_ptr(q), _ptr(out), torch_dtype_code(q), _ptr(k_cache), _ptr(v_cache),
-                                torch_dtype_code(k_cache), _ptr(k_scale), _ptr(v_scale), _ptr(block_table),
-                                _ptr(context_lens), B, Hq, Hkv, D, BLOCK_SIZE, max_blocks, N, max_context_len,
-                                float(scale), _ptr(workspace), ws_bytes, _stream(stream)))
+    out = _decode_out(q, out)
+    check(_front.decode(q, out, k_cache, v_cache, k_scale, v_scale, block_table, context_lens, max_context_len, scale,
+                        num_blocks, workspace, stream))
     return out

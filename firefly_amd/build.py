@@ -17,6 +17,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -82,7 +83,22 @@ def build_library(jobs: int = 8, defines: tuple[str, ...] = (), out: Path | None
     if res.returncode != 0:
         raise RuntimeError(f"link failed: {' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, target)
+    if target == LIB:
+        build_front()
     return target
+
+
+def build_front() -> Path:
+    """The Python front end's CPython extension (csrc/python/front.cpp), next to the library it is bound to at run
+    time (host code only: it names no GPU function and links nothing)."""
+    out = PKG / "_front.so"
+    cxx = os.environ.get("CXX", "g++")
+    cmd = [cxx, "-O2", "-std=c++20", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", f"-I{ROOT / 'include'}",
+           f"-I{sysconfig.get_paths()['include']}", str(CSRC / "python" / "front.cpp"), "-o", str(out)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"front end build failed: {' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
+    return out
 
 
 def build_test_shims() -> None:
