@@ -34,9 +34,6 @@
 //     page of a row has been scored, so a wave never waits on a dependent scalar load between pages.
 #include "mfma_common.h"
 
-#ifndef FFKV_MERGE_ROWS_MIN_BATCH
-#define FFKV_MERGE_ROWS_MIN_BATCH 16  // batches above this merge with paged_decode_mfma_merge_rows
-#endif
 
 #ifndef FFKV_MFMA_MAX_WAVES
 #define FFKV_MFMA_MAX_WAVES 4  // waves (KV heads, or blocks of 16 query heads of one) per workgroup
@@ -844,10 +841,9 @@ void paged_decode_mfma(DecodeArgs a)
 }
 
 // Combine the partials of rows split over several work items.
-// One workgroup of four waves per (row, head): wave w folds segments i_lo + w, i_lo + w + 4, ... into an online
-// (max, denominator, output) state (lane = D/64 dims), then the four states are combined through LDS.
-// MW waves per (row, head): 4 for short piece lists, 16 when rows are few and long (C3-like) and each row has
-// tens of pieces.
+// One workgroup of MW waves per (row, head): wave w folds segments i_lo + w, i_lo + w + MW, ... into an online
+// (max, denominator, output) state (lane = D/64 dims), then the waves' states are combined through LDS.
+// MW waves per (row, head): as many as the rows have pieces for (launch_merge).
 template <int QT, int D, int MW>
 __global__ __launch_bounds__(64 * MW) void paged_decode_mfma_merge(DecodeArgs a)
 {
@@ -940,7 +936,7 @@ __global__ __launch_bounds__(64 * MW) void paged_decode_mfma_merge(DecodeArgs a)
     }
 }
 
-// Combine the partials of split rows when each row has few pieces (more than 16 rows): thread k of the row's
+// Combine the partials of split rows when each row has few pieces: thread k of the row's
 // workgroups owns output dims 4(k % (D/4)) .. +3 of head k / (D/4), folds that chunk of every piece of the row
 // (loads of up to MF = 16 pieces in flight together) and writes it; no cross-thread combine.  Rows written whole by
 // the decode kernel (one piece, no shared-prefix partials) or without tokens are left alone.
@@ -1024,15 +1020,26 @@ int items_m3(const DecodeArgs& a)
     return decode_mfma_items(reinterpret_cast<const void*>(paged_decode_mfma<CT, QT, D>), 64 * sh.nw, sh.gy);
 }
 
-// The merge after a decode launch (rows split over several items, or shared-prefix partials).
+// The merge after a decode launch (rows split over several items, or shared-prefix partials).  A row has about
+// items / batch + 1 pieces (and its prefix chunks).  With many, the pieces of a (row, head) are shared by the waves of a
+// workgroup; with few, one thread folds them all, which reads ahead better but takes another round trip to memory for
+// every 16 pieces and leaves the chip idle where the rows are few.  Whole calls in us, at MW = 16 / 8 / 4 waves / one
+// thread (bf16 pages, 32/8 heads unless given): 24 rows at 8/2 heads of 64 dims (85 pieces) 15.6 / 17.6 / 21.9 / 43.6;
+// 8 rows of 1000 to 2000 tokens (32) 20.4 / 21.1 / 22.8 / 33.8; 17 rows of 100 to 500 (15) 17.9 / 17.4 / 18.3 / 24.8; 32
+// rows (8) 21.0 / 19.5 / 19.8 / 22.9; 64 rows (4) 28.7 / 25.8 / 24.8 / 25.9, of 512 to 4096 tokens 108.7 / 106.1 / 105.1 /
+// 106.1; 128 rows (2) 35.0 / 28.9 / 26.9 / 26.2.  16 rows (16) take 16 waves (27.7 against 27.9 with 8, 256 to 2048
+// tokens), 120 rows over a shared prefix (2 and 4 chunks) one thread (66.8 against 67.0 with 4 waves).
 template <int QT, int D>
-hipError_t launch_merge(const DecodeArgs& a, hipStream_t stream)
+hipError_t launch_merge(const DecodeArgs& a, int items, hipStream_t stream)
 {
-    if (a.batch <= FFKV_MERGE_ROWS_MIN_BATCH)  // few rows over the same items: tens of pieces per row
-    {
-        const dim3 mgrid(static_cast<unsigned>(a.batch), static_cast<unsigned>(a.num_heads));
-        hipLaunchKernelGGL((paged_decode_mfma_merge<QT, D, 16>), mgrid, dim3(1024), 0, stream, a);
-    }
+    const int  pieces = items / a.batch + a.pfx_chunks;
+    const dim3 per_head(static_cast<unsigned>(a.batch), static_cast<unsigned>(a.num_heads));
+    if (pieces >= 16)
+        hipLaunchKernelGGL((paged_decode_mfma_merge<QT, D, 16>), per_head, dim3(1024), 0, stream, a);
+    else if (pieces >= 8)
+        hipLaunchKernelGGL((paged_decode_mfma_merge<QT, D, 8>), per_head, dim3(512), 0, stream, a);
+    else if (pieces >= 4 && a.pfx_chunks == 0)
+        hipLaunchKernelGGL((paged_decode_mfma_merge<QT, D, 4>), per_head, dim3(256), 0, stream, a);
     else
     {
         const dim3 mgrid(static_cast<unsigned>(a.batch), static_cast<unsigned>((a.num_heads * (D / 4) + 255) / 256));
@@ -1052,7 +1059,7 @@ hipError_t launch_m3(const DecodeArgs& a, hipStream_t stream)
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(items), static_cast<unsigned>(gy)), dim3(64 * nw), 0, stream, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_merge<QT, D>(a, stream);
+    return launch_merge<QT, D>(a, items, stream);
 }
 
 template <int CT, int QT>

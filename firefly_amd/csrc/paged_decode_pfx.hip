@@ -91,7 +91,7 @@ hipError_t launch_pfx(const DecodeArgs& a, const PrefillArgs& p, int gy, hipStre
                            dim3(64 * kPfxWaves), 0, stream, a, p);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        return launch_merge<QT, kPfxD>(a, stream);
+        return launch_merge<QT, kPfxD>(a, a.items, stream);
     }
     else
         return hipErrorInvalidConfiguration;  // not reached: decode_pfx_plan declines such builds

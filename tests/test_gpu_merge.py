@@ -1,0 +1,35 @@
+"""The merge of a split decode at the edges of its forms: one thread per output chunk for rows of few pieces, workgroups
+of 4, 8 and 16 waves per (row, head) for more.  A launch has up to 256 work items per pair of 4-head groups here, so the
+batch sizes put the mean number of pieces on both sides of 4, 8 and 16; one long row among short ones has more pieces
+than the mean, and rows of one piece are left to the decode kernel.  Against the CPU checker."""
+
+import math
+
+import numpy as np
+import pytest
+
+import cases
+from test_gpu_parity import _check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B", [1, 16, 17, 32, 33, 64, 65, 130])
+def test_pieces(ff, gpu, B):
+    rng = np.random.default_rng(B)
+    ctx = rng.integers(40, 400, size=B)
+    ctx[B // 2] = 3000
+    ctx[-1] = 0
+    c = cases.make_case(4000 + B, B, 16, 8, 128, ctx, act="bf16", input_scale=1 / math.sqrt(128))
+    _check(ff, gpu, c, 2e-3)
+
+
+@pytest.mark.parametrize("D,kv,act", [(64, "f16", "f16"), (80, "bf16", "bf16"), (256, "bf16", "bf16"),
+                                      (128, "i8", "bf16"), (96, "fp8", "f32")])
+@pytest.mark.parametrize("B", [2, 20, 70])
+def test_pieces_head_dims(ff, gpu, D, kv, act, B):
+    """head_dim 64 and 80 leave lanes of a wave with one dim or none, 256 gives them four."""
+    rng = np.random.default_rng(D + B)
+    c = cases.make_case(4100 + D + B, B, 6, 2, D, rng.integers(1, 900, size=B), act=act, kv=kv,
+                        input_scale=1 / math.sqrt(D))
+    _check(ff, gpu, c, 2e-3 if kv in ("bf16", "f16") else 2e-2)
