@@ -572,6 +572,8 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
         need = lay.acc + parts * head_dim * 4;
     }
 
+    a.cap_tokens = cap;
+    const bool  row = mfma && skip == 0 && ffkv::decode_use_row(a);  // writes no partials
     hipStream_t s = static_cast<hipStream_t>(stream);
     void*       ws = workspace;
     bool        owned = false;
@@ -587,7 +589,11 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
     }
     if (need > 0)
     {
-        if (ws == nullptr)
+        if (ws == nullptr && row)
+        {
+            need = 0;
+        }
+        else if (ws == nullptr)
         {
             hipError_t e = hipMallocAsync(&ws, static_cast<size_t>(need), s);
             if (e != hipSuccess) return hip_fail(e, "decode workspace hipMallocAsync");
@@ -619,7 +625,6 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
     a.ws_acc = need > 0 ? reinterpret_cast<float*>(wsb + lay.acc) : nullptr;
     a.max_blocks = max_blocks;
     a.num_blocks = num_blocks;
-    a.cap_tokens = cap;
     a.chunk = chunk;
     a.max_chunks = max_chunks;
     a.scale_log2 = sm_scale * 1.4426950408889634f;
@@ -676,7 +681,8 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
     }
     if (e == hipSuccess)
         e = fused_pfx ? ffkv::launch_decode_pfx(a, p, plan.gy, s)
-                      : (mfma ? ffkv::launch_decode_mfma(a, s) : ffkv::launch_decode(a, s));
+                      : (row ? ffkv::launch_decode_row(a, s)
+                             : (mfma ? ffkv::launch_decode_mfma(a, s) : ffkv::launch_decode(a, s)));
     if (owned)
     {
         hipError_t fe = hipFreeAsync(ws, s);

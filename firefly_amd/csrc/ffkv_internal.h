@@ -167,6 +167,10 @@ constexpr int kMfmaMaxItems = 2048;
 int decode_mfma_items(const void* kernel, int threads, int grid_y);
 // decode_mfma_items for the kernel instance launch_decode_mfma selects for `a` (its dtypes, head_dim and heads).
 int decode_mfma_launch_items(const DecodeArgs& a);
+// The matrix-core decode in one launch (paged_decode_row.hip), for small batches: whether `a` (sizes and dtypes set)
+// takes it, and its launch (no workspace).
+bool       decode_use_row(const DecodeArgs& a);
+hipError_t launch_decode_row(const DecodeArgs& a, hipStream_t stream);
 bool decode_use_mfma(int cache_dtype, int group, int head_dim);
 
 // Fused shared-prefix decode (paged_decode_pfx.hip): the prefix partials and the decode of the rows' own pages in

@@ -173,13 +173,16 @@ constexpr int kMfmaMaxWaves =
 // One workgroup of a decode launch: work item `item` of `n_items`, KV heads y*nw .. +nw (one per wave; nw waves
 // in the workgroup).  s_v: the workgroup's V tiles in LDS, [nw][16 * D] 16-bit elements.  PW: the page split may
 // weigh the first pfx_items items less (the fused shared-prefix launch); the plain decode's split otherwise.
-template <int CT, int QT, int D, bool PW = false>
+// ROW: the workgroup is one row (item_) and one KV head, or block of 16 of its query heads (y_); its nw_ waves share the
+// row's pages, combine their states through LDS (s_v, as row_lds_bytes sizes it) and write the output: no partials.
+template <int CT, int QT, int D, bool PW = false, bool ROW = false>
 __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_, int n_items_, int nw_, uint16_t* s_v)
 {
+    static_assert(!(PW && ROW), "one split or the other");
     // (the plain decode reads its indices where it uses them: held in registers from the start, they cost the
     // kernel scalar registers it spills)
-    auto item_of = [&]() { return PW ? item_ : static_cast<int>(blockIdx.x); };
-    auto y_of = [&]() { return PW ? y_ : static_cast<int>(blockIdx.y); };
+    auto item_of = [&]() { return PW || ROW ? item_ : static_cast<int>(blockIdx.x); };
+    auto y_of = [&]() { return PW || ROW ? y_ : static_cast<int>(blockIdx.y); };
     // Score products in M (BF: bf16, else f16); PV products in MV.  8-bit codes are exact in both types, so their
     // PV products take f16, where P fits one product (11 bits) instead of a bf16 hi + lo pair; bf16 caches keep
     // bf16 P as hi + lo.  (int8 scores stay f16 with q split in two: bf16 scores, q whole, measured 20 % slower
@@ -253,30 +256,14 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
         return Win{w0, base, uniform(__shfl(incl, 63, 64)), t, n, incl - n, whole};
     };
 
-    // ---- total pages P (every wave on its own, no barriers) -------------------------------------------------
-    // Rows without any token get a zero output and "no pieces" meta here; nothing else touches them.
-    const Win win0 = load_win(0, 0);
-    int       P = 0;
-    for (Win w = win0;;)
+    // The new tokens (fused append) of the rows in `cut`, counted from row r0, to their slots: rows cut short by
+    // max_context_len do not attend them, so no page holding them is staged; one wave copies them, as ffkv_append would.
+    auto copy_cut = [&](uint64_t cut, int r0)
     {
-        if (first_wg && w.w0 + lane < B && w.n == 0)
-        {
-            const int r = w.w0 + lane;
-            if (a.pfx_chunks == 0)  // shared-prefix mode: the merge writes every row
-                for (int e = 0; e < a.num_heads * D; e += 4)
-                    store_out4<QT>(a.out, static_cast<size_t>(r) * a.num_heads * D + e,
-                                   f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-            a.ws_meta[2 * r] = -1;
-            a.ws_meta[2 * r + 1] = -1;
-        }
         if constexpr (kElemBytes<CT> == 2)
-        {
-            // Fused append, rows cut short by max_context_len: their new token is not attended, so no page
-            // holding it is staged; the first wave copies it to its slot here, as ffkv_append would.
-            uint64_t cut = first_wg && a.k_new != nullptr ? __ballot(w.w0 + lane < B && !w.whole) : 0;
             while (cut != 0)
             {
-                const int r = w.w0 + __ffsll(static_cast<long long>(cut)) - 1;
+                const int r = r0 + __ffsll(static_cast<long long>(cut)) - 1;
                 cut &= cut - 1;
                 const int64_t pos = a.context_lens[r];
                 if (pos < 0 || (pos >> 4) >= a.max_blocks) continue;
@@ -292,7 +279,39 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
                         *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.v_new) + src + e);
                 }
             }
+    };
+
+    // ROW: the row's length and its first 64 table entries are loaded together (an entry past the row's pages is never
+    // used), so a row of up to 1024 tokens waits for memory once before its pages go out.
+    int row_toks = 0, row_whole = 0, row_tvec = -1;
+    if constexpr (ROW)
+    {
+        row_tvec = lane < a.max_blocks ? a.block_table[static_cast<int64_t>(item_) * a.max_blocks + lane] : -1;
+        int64_t L = static_cast<int64_t>(a.context_lens[item_]) + 1;  // +1: the token appended this step (:320)
+        row_whole = L <= a.cap_tokens;
+        if (L > a.cap_tokens) L = a.cap_tokens;
+        row_toks = L < 0 ? 0 : static_cast<int>(L);
+        if (a.k_new != nullptr && !row_whole && y_ == 0 && wave == 0) copy_cut(1, item_);
+    }
+
+    // ---- total pages P (every wave on its own, no barriers) -------------------------------------------------
+    // Rows without any token get a zero output and "no pieces" meta here; nothing else touches them.
+    const Win win0 = ROW ? Win{} : load_win(0, 0);
+    int       P = ROW ? (row_toks + kBlockSize - 1) / kBlockSize : 0;
+    if constexpr (!ROW)
+    for (Win w = win0;;)
+    {
+        if (first_wg && w.w0 + lane < B && w.n == 0)
+        {
+            const int r = w.w0 + lane;
+            if (a.pfx_chunks == 0)  // shared-prefix mode: the merge writes every row
+                for (int e = 0; e < a.num_heads * D; e += 4)
+                    store_out4<QT>(a.out, static_cast<size_t>(r) * a.num_heads * D + e,
+                                   f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+            a.ws_meta[2 * r] = -1;
+            a.ws_meta[2 * r + 1] = -1;
         }
+        copy_cut(first_wg && a.k_new != nullptr ? __ballot(w.w0 + lane < B && !w.whole) : 0, w.w0);
         P += w.total;
         if (w.w0 + 64 >= B) break;
         w = load_win(w.w0 + 64, P);
@@ -301,13 +320,14 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
     // PW (fused shared-prefix launch): the first pfx_items items also compute prefix partials, so each of them
     // weighs pfx_share / 1024 of another item: pages [P * cum(i) / T, P * cum(i + 1) / T) with cum(i) = 1024 i -
     // min(i, pfx_items) (1024 - pfx_share) and T = cum(items), as long as that still leaves every item a page.
-    const int     item = item_of();
+    // ROW: wave w of W takes pages [w * P / W, (w + 1) * P / W) of its row, possibly none.
+    const int     item = ROW ? wave : item_of();
     const int     n_items = PW ? n_items_ : static_cast<int>(gridDim.x);
     const int64_t uh = a.pfx_share, up = 1024, H = a.pfx_items;
     const int64_t T_w = H * uh + (n_items - H) * up;
     const bool    weighted = PW && H > 0 && static_cast<int64_t>(P) * min(uh, up) >= T_w;
-    const int     W = weighted ? n_items : min(n_items, P);
-    if (item >= W) return;
+    const int     W = weighted ? n_items : (ROW ? nw_ : min(n_items, P));
+    if (!ROW && item >= W) return;
     auto cum = [&](int64_t i) { return i * up - min(i, H) * (up - uh); };
     const int start = weighted ? static_cast<int>(static_cast<int64_t>(P) * cum(item) / T_w)
                                : static_cast<int>(static_cast<int64_t>(item) * P / W);
@@ -324,8 +344,8 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
     // wave -> (KV head, block of 16 of its query heads): heads kvh * G + h0 + c for c < gc
     const int G = a.group;
     const int HB = (G + 15) >> 4;
-    const int vh = y_of() * (PW ? nw_ : static_cast<int>(blockDim.x) >> 6) + wave;
-    if (vh >= a.num_kv_heads * HB) return;
+    const int vh = ROW ? y_of() : y_of() * (PW ? nw_ : static_cast<int>(blockDim.x) >> 6) + wave;
+    if (!ROW && vh >= a.num_kv_heads * HB) return;
     const int kvh = vh / HB;
     const int h0 = (vh - kvh * HB) * 16;
     const int gc = min(16, G - h0);  // heads of this block
@@ -385,14 +405,19 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
     };
     auto load_tvec = [&](const LRow& r, int tb) { return tb + lane < r.nb ? r.table[tb + lane] : -1; };
 
-    LRow lrow = find_page(start);
+    LRow lrow;
+    if constexpr (ROW)
+        lrow = LRow{item_, 0, P, row_toks, a.block_table + static_cast<int64_t>(item_) * a.max_blocks,
+                    a.k_new != nullptr && row_toks > 0 && row_whole ? (row_toks - 1) & 15 : -1};
+    else
+        lrow = find_page(start);
     int  tb = (start - lrow.pb) & ~63;
-    int  tvec = load_tvec(lrow, tb);
+    int  tvec = ROW && tb == 0 ? row_tvec : load_tvec(lrow, tb);
     LRow lnxt = lrow;
     int  ntvec = -1;
     auto look_ahead = [&]()  // fetch the row after lrow if the item reaches it
     {
-        if (lrow.pb + lrow.nb < end)
+        if (!ROW && lrow.pb + lrow.nb < end)
         {
             lnxt = next_row(lrow);
             ntvec = load_tvec(lnxt, 0);
@@ -404,7 +429,7 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
     // Issue the K and V loads of page lp into r and advance the cursor.
     auto load_next = [&](PageRegs<NW, NWV>& r)
     {
-        if (lp == lrow.pb + lrow.nb)
+        if (!ROW && lp == lrow.pb + lrow.nb)
         {
             lrow = lnxt;
             tb = 0;
@@ -787,12 +812,12 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
         // The scores of page p have consumed Q: a new row's Q is loaded now, ahead of page p + DEPTH's K/V when
         // page p + 1 is already in flight (loads complete in issue order for the wait counter).
         if constexpr (DEPTH > 1)
-            if (row_ends && p + 1 < end) load_q(r[(S + 1) % DEPTH].b);
+            if (!ROW && row_ends && p + 1 < end) load_q(r[(S + 1) % DEPTH].b);
         if (p + DEPTH < end) load_next(cur);
         if constexpr (DEPTH == 1)
-            if (row_ends && p + 1 < end) load_q(cur.b);
+            if (!ROW && row_ends && p + 1 < end) load_q(cur.b);
         if (ok) finish_page(n_tok, tks, tvs, s);
-        if (row_ends || p + 1 == end)
+        if (!ROW && (row_ends || p + 1 == end))
         {
             finish_segment(b, pb, nb, seg_start, p + 1);
             seg_start = p + 1;
@@ -809,6 +834,43 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
             if (p + 1 < end) step.template operator()<1 % DEPTH>(p + 1);
         if constexpr (DEPTH > 2)
             if (p + 2 < end) step.template operator()<2 % DEPTH>(p + 2);
+    }
+
+    // ROW: the waves' states meet in LDS (over their V tiles, once every wave is past its last read of its own): the
+    // accumulators as [wave][head][D], then (max, denominator) as [wave][16]; the block's threads then take four output
+    // dims of a head each.
+    if constexpr (ROW)
+    {
+        float*      s_acc = reinterpret_cast<float*>(s_v);
+        float2*     s_ml = reinterpret_cast<float2*>(s_acc + static_cast<size_t>(nw_) * gc * D);
+        const float l_tot = xor_sum(l_run);
+        __syncthreads();
+        if (c < gc)
+        {
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                *reinterpret_cast<f32x4*>(s_acc + (wave * gc + c) * D + 16 * n + 4 * g) = acc[n] * v_head_scale;
+            if (g == 0) s_ml[wave * 16 + c] = float2{m_run, l_tot};
+        }
+        __syncthreads();
+        for (int k = static_cast<int>(threadIdx.x); k < gc * (D / 4); k += 64 * nw_)
+        {
+            const int h = k / (D / 4);
+            const int d4 = (k - h * (D / 4)) * 4;
+            float     M = kNegInf, L = 0.0f;
+            for (int w = 0; w < nw_; ++w) M = fmaxf(M, s_ml[w * 16 + h].x);
+            const float ref = M == kNegInf ? 0.0f : M;  // no valid page: every weight is 0
+            f32x4       o = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int w = 0; w < nw_; ++w)
+            {
+                const float2 t = s_ml[w * 16 + h];
+                const float  x = __builtin_amdgcn_exp2f(t.x - ref);
+                L += t.y * x;
+                o += *reinterpret_cast<const f32x4*>(s_acc + (w * gc + h) * D + d4) * x;
+            }
+            store_out4<QT>(a.out, (static_cast<size_t>(item_) * a.num_heads + kvh * G + h0 + h) * D + d4,
+                           L > 0.0f ? o * (1.0f / L) : f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+        }
     }
 }
 
