@@ -196,6 +196,20 @@ __device__ __forceinline__ int wave_sum(int x)
     return x;
 }
 
+// Inclusive sum of x over the lanes 0 .. lane, by DPP operands: shifts by 1, 2, 4 and 8 within rows of 16 lanes (lanes
+// shifted in from outside the row read 0), then the last lane of row 0 and 2 to the rows above, then of the lower half to
+// the upper.  Six vector instructions, where __shfl_up steps are six LDS round trips in a chain.  Every lane is active.
+__device__ __forceinline__ int wave_scan(int x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+    return x;
+}
+
 // A value equal in all lanes, moved to a scalar register.
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 

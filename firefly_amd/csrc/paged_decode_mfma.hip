@@ -246,14 +246,8 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
         n = n < 0 ? 0 : n;
         t = t - a.skip_blocks * kBlockSize;
         t = t < 0 ? 0 : t;
-        int incl = n;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1)
-        {
-            const int o = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += o;
-        }
-        return Win{w0, base, uniform(__shfl(incl, 63, 64)), t, n, incl - n, whole};
+        const int incl = wave_scan(n);
+        return Win{w0, base, __builtin_amdgcn_readlane(incl, 63), t, n, incl - n, whole};
     };
 
     // The new tokens (fused append) of the rows in `cut`, counted from row r0, to their slots: rows cut short by
@@ -329,14 +323,23 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
     const int     W = weighted ? n_items : (ROW ? nw_ : min(n_items, P));
     if (!ROW && item >= W) return;
     auto cum = [&](int64_t i) { return i * up - min(i, H) * (up - uh); };
-    const int start = weighted ? static_cast<int>(static_cast<int64_t>(P) * cum(item) / T_w)
-                               : static_cast<int>(static_cast<int64_t>(item) * P / W);
-    const int end = weighted ? static_cast<int>(static_cast<int64_t>(P) * cum(item + 1) / T_w)
-                             : static_cast<int>(static_cast<int64_t>(item + 1) * P / W);
+    // i * P / W; the products of all but very large calls fit 32 bits, whose division is a fraction of the 64-bit one's
+    // (with the scan over a window's rows on DPP steps, 0.5 us off every call: 8 rows of 1000 to 2000 tokens 19.7 -> 19.1 us)
+    auto part = [&](int i)
+    {
+        if (P < (1 << 20)) return static_cast<int>(static_cast<uint32_t>(i) * static_cast<uint32_t>(P) / static_cast<uint32_t>(W));
+        return static_cast<int>(static_cast<int64_t>(i) * P / W);
+    };
+    static_assert(kMfmaMaxItems <= 2048, "items * pages below 2^20 fit 31 bits");
+    const int start = weighted ? static_cast<int>(static_cast<int64_t>(P) * cum(item) / T_w) : part(item);
+    const int end = weighted ? static_cast<int>(static_cast<int64_t>(P) * cum(item + 1) / T_w) : part(item + 1);
     // largest item i with start(i) <= x
     auto last_item = [&](int64_t x) -> int
     {
-        if (!weighted) return static_cast<int>(((x + 1) * W + P - 1) / P - 1);  // largest i with i*P/W <= x
+        if (!weighted && P < (1 << 20))  // largest i with i*P/W <= x
+            return static_cast<int>((static_cast<uint32_t>(x + 1) * static_cast<uint32_t>(W) + static_cast<uint32_t>(P - 1)) /
+                                    static_cast<uint32_t>(P)) - 1;
+        if (!weighted) return static_cast<int>(((x + 1) * W + P - 1) / P - 1);
         const int64_t K = ((x + 1) * T_w + P - 1) / P - 1;                      // cum(i) <= K
         return static_cast<int>(K < H * uh ? K / uh : H + (K - H * uh) / up);
     };
