@@ -19,7 +19,11 @@
 // one (cos, sin) pair of one of them into LDS (inv_freq once per thread, outside the loop), and the tokens' Hq +
 // Hkv head rows are spread over the workgroup, D/16 lanes per row, each lane holding 8 dims of the low half and
 // the matching 8 dims of the high half.  A thread issues the loads of two rows before rotating either, and the
-// first two rows' loads go out before the table's barrier, so the loads overlap the double-precision sin/cos.
+// first rows' loads (and their tokens' page entries) go out before the table is computed, so they overlap the
+// double-precision sin/cos.  Where a workgroup takes one token, only the wave that fills the table evaluates the
+// frequencies (the others used to as well, for nothing): 16 tokens at 32/8 heads 6.3 -> 4.7 us (kernel), 800 tokens 10.1 ->
+// 8.6, 1600 tokens 14.2 -> 13.0, 32000 tokens into int8 pages 165 -> 161.  From 512 or 1024 tokens on several tokens per
+// workgroup (the bulk form) is slower still (1400 tokens at 16/4 heads of 64 dims 10.1 -> 11.2 us).
 #include "ffkv_device.h"
 #include "ffkv_internal.h"
 
@@ -119,11 +123,13 @@ __global__ __launch_bounds__(256) void rope_append_kernel(RopeArgs a)
     // inv_freq of this thread's pair, once (:74-76)
     const int   my_i = threadIdx.x % HALF;
     const int   my_t = threadIdx.x / HALF;  // table row this thread fills (threads beyond TPI rows fill none)
-    const float inv_freq = static_cast<float>(pow(static_cast<double>(a.theta), -2.0 * my_i / D));
+    float       inv_freq = 0.0f;
+    if (my_t < TPI) inv_freq = static_cast<float>(pow(static_cast<double>(a.theta), -2.0 * my_i / D));
 
     for (int64_t tok0 = static_cast<int64_t>(blockIdx.x) * TPI; tok0 < tokens; tok0 += static_cast<int64_t>(gridDim.x) * TPI)
     {
         __syncthreads();  // the previous tokens' rows are done with the table
+        auto fill_table = [&]()
         {
             const int64_t tok = tok0 + my_t;
             if (my_t < TPI && tok < tokens)
@@ -135,16 +141,18 @@ __global__ __launch_bounds__(256) void rope_append_kernel(RopeArgs a)
                 s_cos[my_t][my_i] = static_cast<float>(cos(static_cast<double>(ang)));
                 s_sin[my_t][my_i] = static_cast<float>(sin(static_cast<double>(ang)));
             }
-        }
+        };
 
         // Row u of the iteration: token tok0 + u / rows, head row u % rows (q heads, then kv heads).  Loads of NB
-        // rows go out first (before the table barrier for the first batch), then the rows are rotated and stored.
+        // rows and their page entries go out first (before the table is computed for the first batch), then the rows are
+        // rotated and stored.
         // every thread runs the first batch (possibly without rows) so that all reach the table barrier
         for (int u0 = rsub;; u0 += NB * RPP)
         {
             Raw8 rl[NB], rh[NB], vl[NB], vh[NB];
             bool act[NB], isq[NB];
             int  tl[NB], hh[NB];
+            int  phys[NB], slot[NB];  // page (negative: none) and slot of a k row's token
             size_t rowoff[NB];
 #pragma unroll
             for (int k = 0; k < NB; ++k)
@@ -165,15 +173,28 @@ __global__ __launch_bounds__(256) void rope_append_kernel(RopeArgs a)
                     load_raw8<SRC>(base, rowoff[k] + HALF + 8 * lane, rh[k]);
                     if constexpr (APPEND)
                     {
+                        phys[k] = -1;
+                        slot[k] = 0;
                         if (!isq[k])
                         {
+                            // page slot of the row's token, as the append kernel computes it
+                            const int     b = static_cast<int>(tok / a.seq_len);
+                            const int     t = static_cast<int>(tok % a.seq_len);
+                            const int64_t pos = static_cast<int64_t>(a.context_lens ? a.context_lens[b] : 0) + t;
+                            if (pos >= 0 && (pos >> 4) < a.max_blocks)
+                                phys[k] = a.block_table[static_cast<int64_t>(b) * a.max_blocks + (pos >> 4)];
+                            slot[k] = static_cast<int>(pos & 15);
                             load_raw8<SRC>(a.v, rowoff[k] + 8 * lane, vl[k]);
                             load_raw8<SRC>(a.v, rowoff[k] + HALF + 8 * lane, vh[k]);
                         }
                     }
                 }
             }
-            if (u0 == rsub) __syncthreads();  // the table of these tokens is written (first batch: every thread)
+            if (u0 == rsub)
+            {
+                fill_table();
+                __syncthreads();  // the table of these tokens is written (first batch: every thread)
+            }
 #pragma unroll
             for (int k = 0; k < NB; ++k)
             {
@@ -198,22 +219,11 @@ __global__ __launch_bounds__(256) void rope_append_kernel(RopeArgs a)
                 if constexpr (APPEND)
                 {
                     if (isq[k]) continue;
-                    // page slot of the row's token, as the append kernel computes it
-                    const int64_t tok = tok0 + tl[k];
-                    const int     b = static_cast<int>(tok / a.seq_len);
-                    const int     t = static_cast<int>(tok % a.seq_len);
-                    const int64_t pos = static_cast<int64_t>(a.context_lens ? a.context_lens[b] : 0) + t;
-                    bool          ok = pos >= 0 && (pos >> 4) < a.max_blocks;
-                    int           phys = -1;
-                    if (ok)
-                    {
-                        phys = a.block_table[static_cast<int64_t>(b) * a.max_blocks + (pos >> 4)];
-                        ok = phys >= 0 && phys < a.num_blocks;
-                    }
+                    const bool ok = phys[k] >= 0 && phys[k] < a.num_blocks;
                     // `ok` is per token, the same for the row's LPR lanes (the only ones the int8 reduction reads)
                     if (!ok) continue;
                     const int    h = hh[k];
-                    const size_t dst_row = (static_cast<size_t>(phys) * kBlockSize + (pos & 15)) * a.num_kv_heads + h;
+                    const size_t dst_row = (static_cast<size_t>(phys[k]) * kBlockSize + slot[k]) * a.num_kv_heads + h;
                     // k as stored in its dtype (the values the reference's append would read back)
                     unpack8<SRC>(rl[k], yl);
                     unpack8<SRC>(rh[k], yh);
