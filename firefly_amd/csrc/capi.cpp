@@ -557,11 +557,13 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
     }
     a.cap_tokens = cap;
     const bool row = mfma && skip == 0 && ffkv::decode_use_row(a);  // writes no partials
-    // New tokens (k_new) that the decode itself writes: always into 16-bit pages; quantized ones in the one-launch kernel,
-    // and in the split one unless the call may be so long that the code's cost there (1.5 %) exceeds the append launch.
-    const bool app = k_new != nullptr && mfma && skip == 0 &&
-                     (!quantized(cache_dtype) || row ||
-                      static_cast<int64_t>(batch) * cap * num_kv_heads * head_dim * 2 <= (int64_t{1} << 30));
+    // New tokens (k_new) that the decode itself writes: into fp32 pages, into 16-bit pages on the matrix cores; quantized
+    // ones on the matrix cores, in the one-launch kernel, and in the split one unless the call may be so long that the
+    // code's cost there (1.5 %) exceeds the append launch.
+    const bool app = k_new != nullptr && skip == 0 &&
+                     (!quantized(cache_dtype) ? mfma || cache_dtype == FFKV_DTYPE_F32 :
+                      (mfma && (row || static_cast<int64_t>(batch) * cap * num_kv_heads * head_dim * 2 <=
+                                           (int64_t{1} << 30))));
     if (app)
     {
         a.k_new = k_new;
@@ -731,11 +733,10 @@ int ffkv_append_paged_decode(const void* k_new, const void* v_new, int src_dtype
     if (batch > 0 && (!k_new || !v_new)) return fail(FFKV_ERR_INVALID_ARGUMENT, "null k_new or v_new pointer");
     if (batch > 0 && (!aligned16(k_new) || !aligned16(v_new)))
         return fail(FFKV_ERR_INVALID_ARGUMENT, "k_new and v_new must be 16-byte aligned");
-    // The decode itself writes the new tokens when they already have the cache's 16-bit type, or quantizes them (4 rows of 17
-    // to 255 tokens at 16/8 heads on int8 pages 12.8 -> 8.9 us per step, 16 rows of 256 to 2048 at 32/8 24.3 -> 21.7);
-    // otherwise the append kernel runs first.
-    const bool fused = quantized(cache_dtype) ||
-                       (src_dtype == cache_dtype && (cache_dtype == FFKV_DTYPE_BF16 || cache_dtype == FFKV_DTYPE_F16));
+    // The decode itself writes the new tokens when they already have the cache's type (32 rows on fp32 pages 113.9 -> 111.0
+    // us per step), or quantizes them (4 rows of 17 to 255 tokens at 16/8 heads on int8 pages 12.8 -> 8.9 us per step, 16 rows of
+    // 256 to 2048 at 32/8 24.3 -> 21.7); otherwise the append kernel runs first.
+    const bool fused = quantized(cache_dtype) || src_dtype == cache_dtype;
     if (!fused)
     {
         const int rc = ffkv_append(k_new, v_new, src_dtype, k_cache, v_cache, cache_dtype, k_scale, v_scale,
