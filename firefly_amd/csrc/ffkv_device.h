@@ -432,6 +432,10 @@ __device__ __forceinline__ void load_act4(const void* base, int dt, size_t i, fl
     }
 }
 
+// Factor from a softmax state's accumulator to the output, for denominator l: 0 where there was no key (l == 0), and
+// NaN where l is NaN (a NaN or infinite score among the keys), whichever launches the row was split over.
+__device__ __forceinline__ float softmax_inv(float l, float scale = 1.0f) { return l == 0.0f ? 0.0f : scale / l; }
+
 __device__ __forceinline__ void store_act1(void* base, int dt, size_t i, float x)
 {
     if (dt == F32)

@@ -22,6 +22,9 @@ using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
 using u32x2 = uint32_t __attribute__((ext_vector_type(2)));
 
 constexpr float kNegInf = -__builtin_huge_valf();
+// Seed of a running maximum: no finite score lies below it, and a score of -inf keeps weight 0 beside it (with a seed of
+// -inf it would be 2^(-inf + inf), NaN).  A state without any key is (kLowest, 0, 0).
+constexpr float kLowest = -3.402823466e38f;
 
 // MFMA input element type (bf16 or f16), chosen per cache and q type by kBF below.
 template <bool BF>

@@ -398,7 +398,7 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
         {
             const float lsum = s_l[g];
             store_act1(a.out, a.qo_dtype, (static_cast<size_t>(b) * a.num_heads + hq0 + g) * D + d,
-                       lsum > 0.0f ? acc_v / lsum : 0.0f);
+                       lsum == 0.0f ? 0.0f : acc_v / lsum);
         }
         else
         {
@@ -461,7 +461,7 @@ __global__ __launch_bounds__(256) void paged_decode_merge(DecodeArgs a)
         }
         m = mn;
     }
-    const float  inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const float  inv = softmax_inv(l);
     const size_t ob = (static_cast<size_t>(b) * a.num_heads + h) * D + d4;
 #pragma unroll
     for (int i = 0; i < 4; ++i) store_act1(a.out, a.qo_dtype, ob + i, o[i] * inv);

@@ -644,7 +644,7 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
         }
     };
 
-    float m_run = kNegInf;  // running max of head c (log2 domain), equal in the four lane groups
+    float m_run = kLowest;  // running max of head c (log2 domain), equal in the four lane groups
     float l_run = 0.0f;     // this lane's share of the denominator (tokens 4g..4g+3 of each page)
     f32x4 acc[NT];
 
@@ -825,7 +825,7 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
         {
             if (c < gc)
             {
-                const float inv = l_tot > 0.0f ? v_head_scale / l_tot : 0.0f;
+                const float inv = softmax_inv(l_tot, v_head_scale);
 #pragma unroll
                 for (int n = 0; n < NT; ++n)
                     store_out4<QT>(a.out, (static_cast<size_t>(b) * a.num_heads + h) * D + 16 * n + 4 * g,
@@ -887,7 +887,7 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
         {
             finish_segment(b, pb, nb, seg_start, p + 1);
             seg_start = p + 1;
-            m_run = kNegInf;
+            m_run = kLowest;
             l_run = 0.0f;
 #pragma unroll
             for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -923,19 +923,18 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
         {
             const int h = k / (D / 4);
             const int d4 = (k - h * (D / 4)) * 4;
-            float     M = kNegInf, L = 0.0f;
+            float     M = kLowest, L = 0.0f;
             for (int w = 0; w < nw_; ++w) M = fmaxf(M, s_ml[w * 16 + h].x);
-            const float ref = M == kNegInf ? 0.0f : M;  // no valid page: every weight is 0
-            f32x4       o = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            f32x4     o = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             for (int w = 0; w < nw_; ++w)
             {
                 const float2 t = s_ml[w * 16 + h];
-                const float  x = __builtin_amdgcn_exp2f(t.x - ref);
+                const float  x = __builtin_amdgcn_exp2f(t.x - M);
                 L += t.y * x;
                 o += *reinterpret_cast<const f32x4*>(s_acc + (w * gc + h) * D + d4) * x;
             }
             store_out4<QT>(a.out, (static_cast<size_t>(item_) * a.num_heads + kvh * G + h0 + h) * D + d4,
-                           L > 0.0f ? o * (1.0f / L) : f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+                           o * softmax_inv(L));
         }
     }
 }
@@ -994,7 +993,7 @@ __global__ __launch_bounds__(64 * MW) void paged_decode_mfma_merge(DecodeArgs a)
     // pieces: the shared-prefix partials (slots pfx_slot0 + k * batch + b), then work items i_lo .. i_hi (slots
     // i + b) when the row has pages of its own
     const int pieces = a.pfx_chunks + (i_lo >= 0 ? i_hi - i_lo + 1 : 0);
-    float     m = kNegInf, l = 0.0f, o[PER];
+    float     m = kLowest, l = 0.0f, o[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) o[k] = 0.0f;
     // Wave w folds pieces w, w + MW, ...; the loads of FOLD pieces go out together before any is folded, so a
@@ -1026,7 +1025,7 @@ __global__ __launch_bounds__(64 * MW) void paged_decode_mfma_merge(DecodeArgs a)
 #pragma unroll
         for (int f = 0; f < FOLD; ++f)
         {
-            if (ms[f] == kNegInf) continue;  // segment without a valid page (or past the row's pieces)
+            if (ms[f] == kNegInf && ls[f] == 0.0f) continue;  // past the row's pieces, or a prefix chunk without keys
             const float mn = fmaxf(m, ms[f]);
             const float wa = __builtin_amdgcn_exp2f(m - mn);
             const float wb = __builtin_amdgcn_exp2f(ms[f] - mn);
@@ -1048,21 +1047,18 @@ __global__ __launch_bounds__(64 * MW) void paged_decode_mfma_merge(DecodeArgs a)
     if (threadIdx.x < D)
     {
         const int d = threadIdx.x;
-        float     M = kNegInf;
+        float     M = kLowest;
 #pragma unroll
         for (int w = 0; w < MW; ++w) M = fmaxf(M, s_m[w]);
         float L = 0.0f, O = 0.0f;
-        if (M != kNegInf)
-        {
 #pragma unroll
-            for (int w = 0; w < MW; ++w)
-            {
-                const float wt = __builtin_amdgcn_exp2f(s_m[w] - M);
-                L += s_l[w] * wt;
-                O += s_o[w][d] * wt;
-            }
+        for (int w = 0; w < MW; ++w)
+        {
+            const float wt = __builtin_amdgcn_exp2f(s_m[w] - M);
+            L += s_l[w] * wt;
+            O += s_o[w][d] * wt;
         }
-        store_act1(a.out, QT, ob + d, L > 0.0f ? O / L : 0.0f);
+        store_act1(a.out, QT, ob + d, L == 0.0f ? 0.0f : O / L);
     }
 }
 
@@ -1082,7 +1078,7 @@ __global__ __launch_bounds__(256) void paged_decode_mfma_merge_rows(DecodeArgs a
     const int     h = k / (D / 4);
     const int     d4 = (k - h * (D / 4)) * 4;
     const int     pieces = a.pfx_chunks + (i_lo >= 0 ? i_hi - i_lo + 1 : 0);
-    float         m = kNegInf, l = 0.0f;
+    float         m = kLowest, l = 0.0f;
     f32x4         o = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     for (int i0 = 0; i0 < pieces; i0 += MF)
     {
@@ -1112,7 +1108,7 @@ __global__ __launch_bounds__(256) void paged_decode_mfma_merge_rows(DecodeArgs a
 #pragma unroll
         for (int f = 0; f < MF; ++f)
         {
-            if (ms[f] == kNegInf) continue;  // a piece without a valid page (or past the row's pieces)
+            if (ms[f] == kNegInf && ls[f] == 0.0f) continue;  // past the row's pieces, or a prefix chunk without keys
             const float mn = fmaxf(m, ms[f]);
             const float wa = __builtin_amdgcn_exp2f(m - mn);
             const float wb = __builtin_amdgcn_exp2f(ms[f] - mn);
@@ -1122,7 +1118,7 @@ __global__ __launch_bounds__(256) void paged_decode_mfma_merge_rows(DecodeArgs a
         }
     }
     store_out4<QT>(a.out, (static_cast<size_t>(b) * a.num_heads + h) * D + d4,
-                   l > 0.0f ? o * (1.0f / l) : f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+                   o * softmax_inv(l));
 }
 
 namespace

@@ -1305,7 +1305,7 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
         }
         else if (col_ok[gi])
         {
-            const float  inv = l_tot > 0.0f ? v_head_scale / l_tot : 0.0f;
+            const float  inv = softmax_inv(l_tot, v_head_scale);
             const size_t ob = qrow[gi] * D;
 #pragma unroll
             for (int n = 0; n < NT; ++n) store_out4<QT>(a.out, ob + 16 * n + 4 * g, acc[gi][n] * inv);
@@ -1389,7 +1389,7 @@ __global__ __launch_bounds__(256) void paged_prefill_merge(PrefillArgs a)
     }
     const int    h = grp % Hkv * G + r % G;
     const size_t ob = ((static_cast<size_t>(grp / Hkv) * S + r / G) * a.num_heads + h) * D + 16 * n + 4 * (lane >> 4);
-    store_out4<QT>(a.out, ob, l > 0.0f ? o * (1.0f / l) : f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+    store_out4<QT>(a.out, ob, o * softmax_inv(l));
 }
 
 namespace
