@@ -260,7 +260,8 @@ def append_paged_attention(k_new, v_new, q, k_cache, v_cache, block_table, conte
                            v_scale=None, max_context_len: int = 0, scale: float = 0.0, workspace=None,
                            num_blocks: int | None = None, stream=None):
     """``append_kv_cache(k_new, v_new, ...)`` (one token per row) then ``paged_attention``, as one call
-    (``ffkv_append_paged_decode``; a single launch for 16-bit caches fed in their own dtype)."""
+    (``ffkv_append_paged_decode``; for 16-bit caches fed in their own dtype the decode's launch appends too, and no
+    other row of the call may then attend a row's new slot)."""
     out = _decode_out(q, out)
     check(_front.append_decode(q, out, k_cache, v_cache, k_scale, v_scale, block_table, context_lens, max_context_len,
                                scale, num_blocks, k_new, v_new, workspace, stream))

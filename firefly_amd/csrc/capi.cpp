@@ -491,8 +491,7 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
                 const float* k_scale, const float* v_scale, const int32_t* block_table, const int32_t* context_lens,
                 int batch, int num_heads, int num_kv_heads, int head_dim, int block_size, int max_blocks,
                 int num_blocks, int max_context_len, float scale, int shared_blocks, void* workspace,
-                size_t workspace_bytes, void* stream, const void* k_new = nullptr, const void* v_new = nullptr,
-                int src_dtype = 0)
+                size_t workspace_bytes, void* stream, const void* k_new = nullptr, const void* v_new = nullptr)
 {
     if (block_size != FFKV_BLOCK_SIZE) return fail(FFKV_ERR_UNSUPPORTED, "block_size must be 16, got %d", block_size);
     if (!is_act(qo_dtype)) return fail(FFKV_ERR_UNSUPPORTED, "unsupported q/out dtype %d", qo_dtype);
@@ -555,21 +554,6 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
         a.pfx_items = plan.pfx_items;
         a.pfx_share = plan.pfx_share;
     }
-    a.cap_tokens = cap;
-    const bool row = mfma && skip == 0 && ffkv::decode_use_row(a);  // writes no partials
-    // New tokens (k_new) that the decode itself writes: into fp32 pages, into 16-bit pages on the matrix cores; quantized
-    // ones on the matrix cores, in the one-launch kernel, and in the split one unless the call may be so long that the
-    // code's cost there (1.5 %) exceeds the append launch.
-    const bool app = k_new != nullptr && skip == 0 &&
-                     (!quantized(cache_dtype) ? mfma || cache_dtype == FFKV_DTYPE_F32 :
-                      (mfma && (row || static_cast<int64_t>(batch) * cap * num_kv_heads * head_dim * 2 <=
-                                           (int64_t{1} << 30))));
-    if (app)
-    {
-        a.k_new = k_new;
-        a.v_new = v_new;
-        a.src_dtype = src_dtype;
-    }
     a.items = fused_pfx ? plan.items : (mfma ? ffkv::decode_mfma_launch_items(a) : 0);
 
     // workspace layout: MFMA kernel see mfma_layout, generic kernel [ml | acc] (none for single-chunk rows)
@@ -588,6 +572,8 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
         need = lay.acc + parts * head_dim * 4;
     }
 
+    a.cap_tokens = cap;
+    const bool  row = mfma && skip == 0 && ffkv::decode_use_row(a);  // writes no partials
     hipStream_t s = static_cast<hipStream_t>(stream);
     void*       ws = workspace;
     bool        owned = false;
@@ -677,13 +663,21 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
         p.ws_acc = a.ws_acc;
         if (!fused_pfx) e = ffkv::launch_prefix_partials(p, s);
     }
-    if (k_new != nullptr && !app && e == hipSuccess)
+    if (k_new != nullptr && e == hipSuccess)
     {
-        ffkv::AppendArgs ap{k_new,        v_new,        const_cast<void*>(k_cache), const_cast<void*>(v_cache),
-                            const_cast<float*>(k_scale), const_cast<float*>(v_scale), block_table,
-                            context_lens, src_dtype,    cache_dtype,  batch, 1, num_kv_heads, head_dim,
-                            max_blocks,   num_blocks};
-        e = ffkv::launch_append(ap, s);
+        if (mfma && skip == 0)
+        {
+            a.k_new = k_new;  // the decode kernel writes the step's token into its page and attends it
+            a.v_new = v_new;
+        }
+        else
+        {
+            ffkv::AppendArgs ap{k_new,        v_new,        const_cast<void*>(k_cache), const_cast<void*>(v_cache),
+                                const_cast<float*>(k_scale), const_cast<float*>(v_scale), block_table,
+                                context_lens, cache_dtype,  cache_dtype,  batch, 1, num_kv_heads, head_dim,
+                                max_blocks,   num_blocks};
+            e = ffkv::launch_append(ap, s);
+        }
     }
     if (e == hipSuccess)
         e = fused_pfx ? ffkv::launch_decode_pfx(a, p, plan.gy, s)
@@ -733,10 +727,9 @@ int ffkv_append_paged_decode(const void* k_new, const void* v_new, int src_dtype
     if (batch > 0 && (!k_new || !v_new)) return fail(FFKV_ERR_INVALID_ARGUMENT, "null k_new or v_new pointer");
     if (batch > 0 && (!aligned16(k_new) || !aligned16(v_new)))
         return fail(FFKV_ERR_INVALID_ARGUMENT, "k_new and v_new must be 16-byte aligned");
-    // The decode itself writes the new tokens when they already have the cache's type (32 rows on fp32 pages 113.9 -> 111.0
-    // us per step), or quantizes them (4 rows of 17 to 255 tokens at 16/8 heads on int8 pages 12.8 -> 8.9 us per step, 16 rows of
-    // 256 to 2048 at 32/8 24.3 -> 21.7); otherwise the append kernel runs first.
-    const bool fused = quantized(cache_dtype) || src_dtype == cache_dtype;
+    // One launch when the step's k/v already have the cache's 16-bit type; otherwise the append kernel, then the
+    // decode.
+    const bool fused = src_dtype == cache_dtype && (cache_dtype == FFKV_DTYPE_BF16 || cache_dtype == FFKV_DTYPE_F16);
     if (!fused)
     {
         const int rc = ffkv_append(k_new, v_new, src_dtype, k_cache, v_cache, cache_dtype, k_scale, v_scale,
@@ -749,7 +742,7 @@ int ffkv_append_paged_decode(const void* k_new, const void* v_new, int src_dtype
     }
     return decode_impl(q, out, qo_dtype, k_cache, v_cache, cache_dtype, k_scale, v_scale, block_table, context_lens,
                        batch, num_heads, num_kv_heads, head_dim, block_size, max_blocks, num_blocks, max_context_len,
-                       scale, 0, workspace, workspace_bytes, stream, k_new, v_new, src_dtype);
+                       scale, 0, workspace, workspace_bytes, stream, k_new, v_new);
 }
 
 size_t ffkv_decode_shared_prefix_workspace_bytes(int batch, int num_heads, int num_kv_heads, int head_dim,

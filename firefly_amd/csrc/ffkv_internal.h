@@ -135,13 +135,11 @@ struct DecodeArgs
     // and their share of the rows' own pages is pfx_share / 1024 of another item's.  0 elsewhere.
     int            pfx_items;
     int            pfx_share;
-    // Fused append: [batch, 1, num_kv_heads, head_dim].  16-bit caches, k/v in the cache dtype: the item holding a row's
-    // last page takes the new token from here and writes it to its page slot.  8-bit caches, k/v in src_dtype: that item
-    // quantizes the token into its slot before it loads the page.  (The first wave writes the tokens of rows cut short by
-    // cap_tokens.)
+    // Fused append (16-bit caches, k/v in the cache dtype): [batch, 1, num_kv_heads, head_dim]; the item holding a
+    // row's last page takes the new token from here and writes it to its page slot (the first wave copies the
+    // tokens of rows cut short by cap_tokens).
     const void*    k_new;
     const void*    v_new;
-    int            src_dtype;
 };
 
 hipError_t launch_append(const AppendArgs& a, hipStream_t stream);
@@ -169,7 +167,7 @@ constexpr int kMfmaMaxItems = 2048;
 int decode_mfma_items(const void* kernel, int threads, int grid_y);
 // decode_mfma_items for the kernel instance launch_decode_mfma selects for `a` (its dtypes, head_dim and heads).
 int decode_mfma_launch_items(const DecodeArgs& a);
-// The matrix-core decode in one launch (paged_decode_row.h), for small batches: whether `a` (sizes and dtypes set)
+// The matrix-core decode in one launch (paged_decode_row.hip), for small batches: whether `a` (sizes and dtypes set)
 // takes it, and its launch (no workspace).
 bool       decode_use_row(const DecodeArgs& a);
 hipError_t launch_decode_row(const DecodeArgs& a, hipStream_t stream);

@@ -69,23 +69,6 @@ __device__ __forceinline__ void load_row8(const void* base, size_t row, int D, i
     }
 }
 
-template <int CT>
-__device__ __forceinline__ void store_row8(void* base, size_t row, int D, int lane, const Raw8& r)
-{
-    if constexpr (CT == F32)
-    {
-        float* p = static_cast<float*>(base) + row * D;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-            *reinterpret_cast<u32x4*>(p + lane_dim<CT>(D, lane, 4 * h)) =
-                u32x4{r.w[4 * h], r.w[4 * h + 1], r.w[4 * h + 2], r.w[4 * h + 3]};
-    }
-    else
-    {
-        store_raw8<CT>(base, row * D + lane * 8, r);
-    }
-}
-
 __device__ __forceinline__ int row_tokens(const DecodeArgs& a, int b)
 {
     int64_t L = static_cast<int64_t>(a.context_lens[b]) + 1;  // +1: the token appended this step (:320)
@@ -121,33 +104,6 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
     const int begin = chunk_id * a.chunk;
     const int end = min(begin + a.chunk, L);
     const int G = a.group;
-
-    // Fused append (k_new in fp32, as the cache): the chunk that holds the row's last token takes it from k_new /
-    // v_new and writes it to its slot (j_new, else -1); the token of a row cut short by cap_tokens is written by the
-    // row's first chunk, unattended.
-    // (fp32 caches only: on 16-bit pages of 88 dims the code in the loop cost more than the append launch, 78.7 -> 85.2 us)
-    constexpr bool APP = CT == F32;
-    const size_t   new_row = static_cast<size_t>(b) * a.num_kv_heads + kvh;
-    int            j_new = -1;
-    if (APP && a.k_new != nullptr)
-    {
-        const int ctx = a.context_lens[b];
-        if (ctx >= 0 && ctx < L)
-            j_new = ctx;
-        else if (ctx >= 0 && chunk_id == 0 && (ctx >> 4) < a.max_blocks && tid < LPT && act)
-        {
-            const int ph = a.block_table[static_cast<int64_t>(b) * a.max_blocks + (ctx >> 4)];
-            if (ph >= 0 && ph < a.num_blocks)
-            {
-                const size_t dst = (static_cast<size_t>(ph) * kBlockSize + (ctx & 15)) * a.num_kv_heads + kvh;
-                Raw8         w;
-                load_row8<CT, false>(a.k_new, new_row, D, lane, w);
-                store_row8<CT>(const_cast<void*>(a.k_cache), dst, D, lane, w);
-                load_row8<CT, false>(a.v_new, new_row, D, lane, w);
-                store_row8<CT>(const_cast<void*>(a.v_cache), dst, D, lane, w);
-            }
-        }
-    }
 
     float q[GP][8];
 #pragma unroll
@@ -231,18 +187,8 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
                 ks[u] = vs[u] = 1.0f;
                 if (valid[u] && act)
                 {
-                    if (APP && base + u * TPI + slot == j_new)
-                    {
-                        load_row8<CT, false>(a.k_new, new_row, D, lane, kr[u]);
-                        load_row8<CT, false>(a.v_new, new_row, D, lane, vr[u]);
-                        store_row8<CT>(const_cast<void*>(a.k_cache), row[u], D, lane, kr[u]);
-                        store_row8<CT>(const_cast<void*>(a.v_cache), row[u], D, lane, vr[u]);
-                    }
-                    else
-                    {
-                        load_row8<CT, NT>(a.k_cache, row[u], D, lane, kr[u]);
-                        load_row8<CT, NT>(a.v_cache, row[u], D, lane, vr[u]);
-                    }
+                    load_row8<CT, NT>(a.k_cache, row[u], D, lane, kr[u]);
+                    load_row8<CT, NT>(a.v_cache, row[u], D, lane, vr[u]);
                     if constexpr (CT == I8)
                     {
                         ks[u] = a.k_scale[row[u]];

@@ -175,12 +175,10 @@ constexpr int kMfmaMaxWaves =
 // weigh the first pfx_items items less (the fused shared-prefix launch); the plain decode's split otherwise.
 // ROW: the workgroup is one row (item_) and one KV head, or block of 16 of its query heads (y_); its nw_ waves share the
 // row's pages, combine their states through LDS (s_v, as row_lds_bytes sizes it) and write the output: no partials.
-// APP: the launch may carry new tokens for an 8-bit cache (k_new set), which it quantizes into their pages.
-template <int CT, int QT, int D, bool PW = false, bool ROW = false, bool APP = false>
+template <int CT, int QT, int D, bool PW = false, bool ROW = false>
 __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_, int n_items_, int nw_, uint16_t* s_v)
 {
     static_assert(!(PW && ROW), "one split or the other");
-    static_assert(!APP || kElemBytes<CT> == 1, "16-bit caches take their new tokens from k_new in any launch");
     // (the plain decode reads its indices where it uses them: held in registers from the start, they cost the
     // kernel scalar registers it spills)
     auto item_of = [&]() { return PW || ROW ? item_ : static_cast<int>(blockIdx.x); };
@@ -252,64 +250,19 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
         return Win{w0, base, __builtin_amdgcn_readlane(incl, 63), t, n, incl - n, whole};
     };
 
-    // Fused append into an 8-bit cache: quantize row b's new K and V of KV head h into slot `sl` of page `phys`, byte for
-    // byte as the append kernel does (8 values per lane, K in the first lanes and V in the next; int8: the row's scale
-    // from its absolute maximum).
-    auto append_codes = [&](int b, int h, int phys, int sl)
-    {
-        if constexpr (APP)
-        {
-            constexpr int LPR = D <= 64 ? 8 : (D <= 128 ? 16 : 32);  // lanes per row, those past D / 8 idle
-            const int     idx = lane % LPR;
-            const bool    is_v = lane / LPR == 1;
-            const bool    act = lane < 2 * LPR && 8 * idx < D;
-            float         x[8] = {};
-            if (act)
-                load_act8(is_v ? a.v_new : a.k_new, a.src_dtype,
-                          (static_cast<size_t>(b) * a.num_kv_heads + h) * D + 8 * idx, x);
-            const size_t row = (static_cast<size_t>(phys) * kBlockSize + sl) * a.num_kv_heads + h;
-            float*       scales = const_cast<float*>(is_v ? a.v_scale : a.k_scale);
-            float        sc = 1.0f;
-            if constexpr (CT == I8)
-            {
-                float amax = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                {
-                    const float v = __builtin_fabsf(x[i]);
-                    amax = v > amax ? v : amax;  // NaN never compares greater: ignored
-                }
-                amax = group_max<LPR>(amax);
-                sc = amax == 0.0f ? 1.0f : amax / 127.0f;  // an all-zero row gives codes 0 either way
-                if (act && idx == 0) scales[row] = amax == 0.0f ? 0.0f : sc;
-            }
-            else
-            {
-                sc = scales[h];
-            }
-            uint32_t w[2];
-            quant8<CT == I8>(x, sc, w);
-            if (act)
-                *reinterpret_cast<u32x2*>(static_cast<char*>(const_cast<void*>(is_v ? a.v_cache : a.k_cache)) + row * D +
-                                          8 * idx) = u32x2{w[0], w[1]};
-        }
-    };
-
     // The new tokens (fused append) of the rows in `cut`, counted from row r0, to their slots: rows cut short by
-    // max_context_len do not attend them, so no page holding them is staged; one wave writes them, as ffkv_append would.
+    // max_context_len do not attend them, so no page holding them is staged; one wave copies them, as ffkv_append would.
     auto copy_cut = [&](uint64_t cut, int r0)
     {
-        if constexpr (kElemBytes<CT> == 2 || APP)
-        while (cut != 0)
-        {
-            const int r = r0 + __ffsll(static_cast<long long>(cut)) - 1;
-            cut &= cut - 1;
-            const int64_t pos = a.context_lens[r];
-            if (pos < 0 || (pos >> 4) >= a.max_blocks) continue;
-            const int phys = a.block_table[static_cast<int64_t>(r) * a.max_blocks + (pos >> 4)];
-            if (phys < 0 || phys >= a.num_blocks) continue;
-            if constexpr (kElemBytes<CT> == 2)
+        if constexpr (kElemBytes<CT> == 2)
+            while (cut != 0)
             {
+                const int r = r0 + __ffsll(static_cast<long long>(cut)) - 1;
+                cut &= cut - 1;
+                const int64_t pos = a.context_lens[r];
+                if (pos < 0 || (pos >> 4) >= a.max_blocks) continue;
+                const int phys = a.block_table[static_cast<int64_t>(r) * a.max_blocks + (pos >> 4)];
+                if (phys < 0 || phys >= a.num_blocks) continue;
                 const size_t dst = (static_cast<size_t>(phys) * kBlockSize + (pos & 15)) * a.num_kv_heads * D;
                 const size_t src = static_cast<size_t>(r) * a.num_kv_heads * D;
                 for (int e = 8 * lane; e < a.num_kv_heads * D; e += 8 * 64)
@@ -320,11 +273,6 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
                         *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.v_new) + src + e);
                 }
             }
-            else if constexpr (APP)
-            {
-                for (int h = 0; h < a.num_kv_heads; ++h) append_codes(r, h, phys, static_cast<int>(pos & 15));
-            }
-        }
     };
 
     // ROW: the row's length and its first 64 table entries are loaded together (an entry past the row's pages is never
@@ -507,17 +455,6 @@ __device__ __forceinline__ void decode_wg(const DecodeArgs& a, int item_, int y_
         r.ok = phys >= 0 && phys < a.num_blocks;  // uniform: a masked page is skipped
         r.ns = pg == lrow.nb - 1 ? lrow.ns : -1;  // fused append: the new token sits in the row's last page
         if (!r.ok) return;
-        if constexpr (APP)
-            if (r.ns >= 0)
-            {
-                // Fused append into an 8-bit page: the codes are written first and the page loaded after them (the wave's
-                // stores have reached the caches it loads through once its counter is down).  Every block of 16 query
-                // heads of the KV head writes them, the same bytes, so that each reads its own.
-                append_codes(lrow.b, kvh, phys, r.ns);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            }
         const size_t row_c = (static_cast<size_t>(phys) * kBlockSize + c) * a.num_kv_heads + kvh;
         if constexpr (CT == I8)
         {
@@ -947,9 +884,7 @@ static __device__ uint64_t g_decode_timeline[2 * kTimelineWaves];
 #endif
 
 // Work item blockIdx.x of gridDim.x; KV heads blockIdx.y * NW .. +NW, one per wave (NW = blockDim.x / 64).
-// APP: with new tokens to quantize into an 8-bit cache (a kernel of its own: the code costs the others registers and 1.5 %
-// of their time, 87.3 -> 88.9 us over 48 rows on fp8 pages).
-template <int CT, int QT, int D, bool APP>
+template <int CT, int QT, int D>
 __global__ __launch_bounds__((64 * kMfmaMaxWaves<CT, D>)) __attribute__((amdgpu_waves_per_eu(kMfmaWaves<CT, QT, D>, 8)))
 void paged_decode_mfma(DecodeArgs a)
 {
@@ -957,8 +892,8 @@ void paged_decode_mfma(DecodeArgs a)
 #if FFKV_DECODE_TIMELINE
     const uint64_t t_start = __builtin_amdgcn_s_memrealtime();
 #endif
-    decode_wg<CT, QT, D, false, false, APP>(a, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y),
-                                            static_cast<int>(gridDim.x), static_cast<int>(blockDim.x) >> 6, s_v);
+    decode_wg<CT, QT, D>(a, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), static_cast<int>(gridDim.x),
+                         static_cast<int>(blockDim.x) >> 6, s_v);
 #if FFKV_DECODE_TIMELINE
     const uint64_t t_end = __builtin_amdgcn_s_memrealtime();
     const int      lane = static_cast<int>(threadIdx.x) & 63;
@@ -1139,21 +1074,11 @@ MfmaShape mfma_shape(const DecodeArgs& a)
     return MfmaShape{nw, (vh + nw - 1) / nw};
 }
 
-using MfmaKernel = void (*)(DecodeArgs);
-
-template <int CT, int QT, int D>
-MfmaKernel mfma_kernel(const DecodeArgs& a)
-{
-    if constexpr (kElemBytes<CT> == 1)
-        if (a.k_new != nullptr) return paged_decode_mfma<CT, QT, D, true>;
-    return paged_decode_mfma<CT, QT, D, false>;
-}
-
 template <int CT, int QT, int D>
 int items_m3(const DecodeArgs& a)
 {
     const MfmaShape sh = mfma_shape<CT, D>(a);
-    return decode_mfma_items(reinterpret_cast<const void*>(mfma_kernel<CT, QT, D>(a)), 64 * sh.nw, sh.gy);
+    return decode_mfma_items(reinterpret_cast<const void*>(paged_decode_mfma<CT, QT, D>), 64 * sh.nw, sh.gy);
 }
 
 // The merge after a decode launch (rows split over several items, or shared-prefix partials).  A row has about
@@ -1189,7 +1114,7 @@ hipError_t launch_m3(const DecodeArgs& a, hipStream_t stream)
 {
     const MfmaShape sh = mfma_shape<CT, D>(a);
     const int       nw = sh.nw, gy = sh.gy;
-    const auto      kern = mfma_kernel<CT, QT, D>(a);
+    const auto      kern = paged_decode_mfma<CT, QT, D>;
     // the workspace holds items + batch partial slots
     const int items = a.items > 0 ? a.items : items_m3<CT, QT, D>(a);
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(items), static_cast<unsigned>(gy)), dim3(64 * nw), 0, stream, a);

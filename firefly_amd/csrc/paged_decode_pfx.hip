@@ -16,8 +16,6 @@
 #include "paged_decode_mfma.hip"
 #undef FFKV_DEVICE_BODIES_ONLY
 
-#include "paged_decode_row.h"
-
 #include <cstdlib>
 
 namespace ffkv

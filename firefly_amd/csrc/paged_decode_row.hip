@@ -1,12 +1,13 @@
-// paged_decode_row.h - the matrix-core decode of a small batch in one launch: a workgroup per row and KV head.
+// paged_decode_row.hip - the matrix-core decode of a small batch in one launch: a workgroup per row and KV head.
 //
 // The split decode (paged_decode_mfma.hip) deals the pages of all rows evenly over the chip and folds the pieces of
 // each row with a second kernel.  That pays once there is enough to stream; a small batch of short rows pays more for the
 // second launch, the partials and the search for its rows than for its pages.  Here a workgroup of eight waves takes one
 // row and one KV head (or block of 16 of its query heads): its waves stream shares of the row's pages with the same code
 // (decode_wg with ROW), meet in LDS and write the output.
-// (Compiled as part of paged_decode_pfx.hip, which has the decode's body too.)
-#pragma once
+#define FFKV_DEVICE_BODIES_ONLY 1
+#include "paged_decode_mfma.hip"
+#undef FFKV_DEVICE_BODIES_ONLY
 
 namespace ffkv
 {
@@ -27,13 +28,12 @@ constexpr int row_lds_bytes(int heads)
 }
 static_assert(row_lds_bytes<256>(16) <= 160 * 1024, "a workgroup's LDS fits a CU");
 
-// APP: with new tokens to quantize into an 8-bit cache (as paged_decode_mfma).
-template <int CT, int QT, int D, bool APP>
+template <int CT, int QT, int D>
 __global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(2, 8)))
 void paged_decode_row(DecodeArgs a)
 {
     extern __shared__ __align__(16) uint8_t s_row[];
-    decode_wg<CT, QT, D, false, true, APP>(a, static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.x), 0, kRowWaves,
+    decode_wg<CT, QT, D, false, true>(a, static_cast<int>(blockIdx.y), static_cast<int>(blockIdx.x), 0, kRowWaves,
                                       reinterpret_cast<uint16_t*>(s_row));
 }
 
@@ -43,10 +43,7 @@ hipError_t launch_row3(const DecodeArgs& a, hipStream_t stream)
     const int  hb = (a.group + 15) / 16;
     const int  lds = row_lds_bytes<D>(a.group < 16 ? a.group : 16);
     const dim3 grid(static_cast<unsigned>(a.num_kv_heads * hb), static_cast<unsigned>(a.batch));
-    MfmaKernel kern = paged_decode_row<CT, QT, D, false>;
-    if constexpr (kElemBytes<CT> == 1)
-        if (a.k_new != nullptr) kern = paged_decode_row<CT, QT, D, true>;
-    hipLaunchKernelGGL(kern, grid, dim3(64 * kRowWaves), static_cast<unsigned>(lds), stream, a);
+    hipLaunchKernelGGL((paged_decode_row<CT, QT, D>), grid, dim3(64 * kRowWaves), static_cast<unsigned>(lds), stream, a);
     return hipGetLastError();
 }
 

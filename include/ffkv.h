@@ -150,13 +150,11 @@ FFKV_API int ffkv_paged_decode_noalloc(const void* q, void* out, int qo_dtype, c
  * ffkv_append of one token per row (seq_len 1) followed by ffkv_paged_decode, as one call: the decode step of
  * the reference's model (src/model/qwen_model.cu:138-146, append launch then kernels::attention).  k_new / v_new
  * [batch, 1, num_kv_heads, head_dim] in src_dtype; the other arguments as for the two functions.  When the
- * step's k/v already have the cache's float type there is no append launch (but for 16-bit caches at the head
- * dims of the vector kernel): the decode work item that holds a row's last page reads the new token from k_new /
- * v_new instead of the page, attends it, and writes it to its page slot (rows cut short by max_context_len get
- * the token copied to its slot without attending it).  For I8 and FP8_E4M3 caches the work item quantizes the
- * token into its slot before it reads the page, unless the call's bound on cached bytes (batch * row bound)
- * passes 1 GiB or head_dim takes the vector kernel.  A row's slot for its new token is its own: no other row of
- * the call may attend it.
+ * step's k/v already have the cache's 16-bit type it is a single launch: the decode work item that holds a
+ * row's last page reads the new token from k_new / v_new instead of the page, attends it, and writes it to its
+ * page slot (rows cut short by max_context_len get the token copied to its slot without attending it).  In that
+ * form a row's slot for its new token is its own: no other row of the call may attend it (rows that do, such as
+ * several tokens of one sequence, take ffkv_append and ffkv_paged_decode).
  * Otherwise it runs the two functions in turn.  Either way the pages are
  * bit-identical to ffkv_append's and the output is ffkv_paged_decode's on them.  No counterpart in the
  * reference (two launches there).

@@ -82,7 +82,8 @@ FIREFLY_API void attention_shared_prefix(Tensor& q, Tensor& k_cache, Tensor& v_c
  * @brief The decode step's append_kv_cache(k, v, ...) followed by the decode branch of attention(q, ...), as one
  * call (ffkv_append_paged_decode): k / v [B, 1, kv_head_num, head_dim] are the step's new tokens, written to the
  * pages at context_lens[b] exactly as append_kv_cache writes them, and q [B, 1, Hq, head_dim] attends
- * context_lens[b] + 1 keys.  One kernel launch when k / v have the cache's 16-bit dtype, the two calls otherwise.
+ * context_lens[b] + 1 keys.  One kernel launch when k / v have the cache's 16-bit dtype, the two calls otherwise; no
+ * other row of the call may attend a row's new slot in that launch (such rows take the two calls).
  * The reference runs the pair as two launches (src/model/qwen_model.cu:138-146); 16-bit caches only here (the
  * quantized caches take the scale-taking append_kv_cache and attention overloads).
  */
