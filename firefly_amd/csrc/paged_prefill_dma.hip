@@ -259,14 +259,15 @@ __device__ __forceinline__ void wait_vm()
     __builtin_amdgcn_s_waitcnt(VM | (0x7 << 4) | (0xF << 8));  // vmcnt(VM), expcnt and lgkmcnt not waited on
 }
 
-// Pieces that a row block of `steps` steps is split into (a.n_split > 1), the same in every workgroup of the call:
+// Pieces that a block of `steps` steps, of a row whose last block has `row_steps`, is split into (a.n_split > 1):
 // as many as keep a piece at kPrefillSplitMin steps or more and all pieces of the call together at about split_slots
-// (the workgroups resident at once).  The call's steps are summed over its rows at the middle of their chunks.
+// (the workgroups resident at once).  The call's steps are summed over its rows at the middle of their chunks.  A row is
+// split in all its blocks or in none: the blocks left whole beside split ones would last the longest.
 template <int KP>
-__device__ __forceinline__ int split_pieces(const PrefillArgs& a, int steps, int nrb, int lane)
+__device__ __forceinline__ int split_pieces(const PrefillArgs& a, int steps, int row_steps, int nrb, int lane)
 {
     constexpr int KEYS = KP * kBlockSize;
-    if (steps < a.split_from) return 1;
+    if (row_steps < a.split_from) return 1;
     int64_t total = 0;
     for (int b0 = 0; b0 < a.batch; b0 += 64)
     {
@@ -485,7 +486,10 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
     int64_t part = -1;  // slot of this piece's partials, or -1: the workgroup has all the keys and writes the output
     if (!PFX && nsp > 1)
     {
-        const int np = split_pieces<KP>(a, (pg_hi + KP - 1) / KP, nrb, lane);
+        int64_t row_keys = ctx + S;
+        row_keys = row_keys > L ? L : (row_keys < 0 ? 0 : row_keys);
+        const int row_steps = static_cast<int>((row_keys + KP * kBlockSize - 1) / (KP * kBlockSize));
+        const int np = split_pieces<KP>(a, (pg_hi + KP - 1) / KP, row_steps, nrb, lane);
         if (piece >= np) return;  // uniform over the workgroup
         const int64_t blk = static_cast<int64_t>(grp0) * nrb + rb;
         if (piece == 0 && tid == 0) a.ws_pieces[blk] = np;
@@ -1530,12 +1534,19 @@ hipError_t launch_pfd(const PrefillArgs& a, hipStream_t stream)
 }  // namespace
 
 // A prefill with fewer blocks of 128 query rows than workgroups fit the chip at once leaves it partly idle, and its
-// duration is the longest block's: one request's 256 tokens over 7.9k cached ones at 32 / 8 heads are 64 blocks of 132
+// duration is the longest block's: one request's 256 tokens over 7.9k cached ones at 32 / 8 heads are 64 blocks of 128
 // steps on 64 of 256 CUs.  With k times the blocks resident at once, each block is split into k pieces (223 -> 62 us for
 // that call, of which 7.5 us are the merge; 4 pieces took 75 us, 16 took 61, 32 took 69).  A piece's partials (64 KiB at
-// head_dim 128) and the merge cost about as much as 5 steps, so short blocks stay whole: at 4 and more pieces, 16 steps
-// gain (40 -> 28 us), 8 lose (a 500-token prompt: 19.7 -> 23.4 us); at two pieces, which only put a second workgroup on
-// each CU, 31 steps gain (67.8 -> 62.4 us) and 16 lose (30.7 -> 34.7 us).
+// head_dim 128) and the merge cost about as much as 5 steps, and at two pieces a split only puts a second workgroup on
+// each CU, so short calls stay whole.  Whole -> split in us, 32 / 8 heads of 128 dims, by the steps of the last block:
+//   8 pieces (one request's 256 tokens)   8: 20.4 -> 21.5, 10: 23.4 -> 22.8, 12: 26.2 -> 23.5, 16: 32.6 -> 26.0
+//   32 pieces (64 tokens)                 8: 19.8 -> 18.7,  9: 21.3 -> 17.6, 12: 26.4 -> 19.5
+//   4 pieces (512 tokens; 3 x 160)       13: 28.6 -> 30.5, 14: 30.2 -> 30.6, 15: 31.2 -> 31.1, 16: 32.8 -> 31.7
+//   2 pieces (3 x 256; 8 x 128)          18: 38.5 -> 41.0, 20: 40.4 -> 41.4, 22: 43.8 -> 43.2, 25: 48.8 -> 46.6
+// The host knows only the bound on a row (max_context_len, or the table's width): a call whose bound is below the point
+// where a split gains is not planned for one.  A planned call pays for the merge's launch whatever its rows turn out to
+// be (2.2 to 3.4 us: a first chunk of 256 tokens behind a wide table 13.3 -> 15.8), so its rows are split from a little
+// earlier on (split_from), where that costs no more than the empty merge.
 void prefill_plan(PrefillArgs& a)
 {
     a.n_split = 1;
@@ -1546,13 +1557,12 @@ void prefill_plan(PrefillArgs& a)
     const int           slots = decode_mfma_items(k.fn, k.threads, 1);
     if (blocks <= 0 || 2 * blocks > slots) return;
     int64_t       n = slots / blocks;
-    const int     from = n >= 4 ? 12 : (n == 3 ? 16 : 24);
     const int64_t steps = (static_cast<int64_t>(a.cap_tokens) + k.keys - 1) / k.keys;  // most steps of a block
-    if (steps < from) return;
+    if (steps < (n >= 5 ? 12 : (n >= 3 ? 15 : 24))) return;
+    a.split_from = n >= 8 ? 8 : (n >= 5 ? 9 : (n >= 3 ? 13 : 19));
     n = std::min(std::min(n, steps / kPrefillSplitMin), static_cast<int64_t>(kPrefillSplitMax));
     a.n_split = static_cast<int>(n);
     a.split_slots = slots;
-    a.split_from = from;
 }
 
 PrefillSplitLayout prefill_split_layout(const PrefillArgs& a)

@@ -3,8 +3,9 @@ the unsplit call.
 
 Bar against the closed form as in test_gpu_prefill.py.  Split and unsplit differ by the order of fp32 sums and the
 reference maxima of P's rounding to 11 bits: both lie within the bar, so their difference is held to the sum of two.
-Each case says whether the library splits it (``ffkv_prefill_workspace_bytes``), at the edges of the rule: 12 steps of
-64 keys at four pieces and more, 24 at two.
+Each case says whether the library plans to split it (``ffkv_prefill_workspace_bytes``) at the edges of the rule on the
+bound of a row (12 steps of 64 keys at five pieces and more), or, behind a wide table, whether its rows are split at the
+edges of the rule on their own length (8 steps at eight pieces and more, 9 from five, 13 from three, 19 at two).
 """
 
 import numpy as np
@@ -82,6 +83,50 @@ def test_split_prompt(ff, gpu, S, Hq, Hkv, splits):
     got, whole, ref, split = _both(ff, gpu, c, qn, True)
     assert split == splits
     _check(got, ref, c.act, 2e-3)
+
+
+def _pieces(ff, dev, c, qn, max_context_len=0):
+    """(output, pieces of every block or None) of the case's chunk behind a table of 300 blocks, over a workspace that
+    holds all ones before the call."""
+    import torch
+
+    wide = np.full((c.B, 300), -1, dtype=np.int32)
+    wide[:, :c.max_blocks] = c.block_table
+    q = gu.to_dev(qn, c.act, dev)
+    kp, vp = gu.to_dev(c.k_pool, c.kv, dev), gu.to_dev(c.v_pool, c.kv, dev)
+    bt, cx = torch.from_numpy(wide).to(dev), torch.from_numpy(c.ctx).to(dev)
+    B, S, Hq, D = q.shape
+    out = torch.full((B, S, Hq * D), float("nan"), dtype=q.dtype, device=dev)
+    qt, ct = ff.torch_dtype_code(q), ff.torch_dtype_code(kp)
+    need = ff.lib.ffkv_prefill_workspace_bytes(qt, ct, B, S, Hq, c.Hkv, D, 1, 300, max_context_len)
+    ws = torch.full((max(need, 256),), 255, dtype=torch.uint8, device=dev)
+    ff.check(ff.lib.ffkv_paged_prefill_ws(ff._ptr(q), ff._ptr(out), qt, ff._ptr(kp), ff._ptr(vp), ct, None, None,
+                                          ff._ptr(bt), ff._ptr(cx), B, S, Hq, c.Hkv, D, 16, 300, c.num_blocks,
+                                          max_context_len, 0.0, ff._ptr(ws), ws.numel(), ff._stream(None)))
+    torch.cuda.synchronize()
+    blocks = B * c.Hkv * ((S * Hq // c.Hkv + 127) // 128)
+    return out.float().cpu().numpy(), None if need == 0 else ws[:4 * blocks].view(torch.int32).cpu().numpy()
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,rule", [(1, 32, 8, 33, 8), (1, 32, 8, 256, 8), (1, 32, 8, 350, 9), (3, 32, 8, 160, 13),
+                                             (3, 32, 8, 256, 19)])
+def test_wide_table(ff, gpu, B, Hq, Hkv, S, rule):
+    """32, 8, 5, 4 and 2 pieces planned for: rows one step short of the rule are whole, rows at it are split in every block
+    (all have more than four steps), and a bound below the rule's own plans nothing."""
+    for steps in (rule - 1, rule):
+        ctx = [64 * steps - S] + [0] * (B - 1)
+        c, qn = _case(1000 + S + steps, B, Hq, Hkv, 128, ctx, S)
+        # the pools hold the chunk's keys as well: nothing is appended
+        ref = O.paged_prefill_f64(qn, c.act, c.k_pool, c.v_pool, c.kv, c.block_table, c.ctx)
+        got, pieces = _pieces(ff, gpu, c, qn)
+        _check(got.reshape(ref.shape), ref, c.act, 2e-3)
+        row0 = pieces.reshape(B, -1)[0]
+        assert (row0 > 1).any() == (steps == rule) and (pieces >= 1).all()
+        if steps == rule:
+            assert row0.min() >= 2
+        assert (pieces.reshape(B, -1)[1:] == 1).all()
+        got, pieces = _pieces(ff, gpu, c, qn, max_context_len=64 * 11)
+        assert pieces is None
 
 
 def test_split_prefill_reuses_scratch(ff, gpu):
