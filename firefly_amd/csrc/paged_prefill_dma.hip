@@ -319,7 +319,9 @@ struct PrefillLds
 // S3 bytes) and `s_vover` an int in LDS.  Every wave of the workgroup calls it; it leaves no load in flight into
 // the stages.  (paged_prefill_dma gives each stage an LDS array of its own, which tells the compiler that they
 // do not overlap.)
-template <int QT, int D, int CT, bool PFX, int RG>
+// SPLIT: a prefill split over its keys (a.n_split > 1), in instances of its own: the pieces cost a workgroup ten scalar
+// registers, which calls that are not split paid for too (int8 at head_dim 64, 15 x 490 tokens over 1500: 216.8 -> 218.7 us).
+template <int QT, int D, int CT, bool PFX, int RG, bool SPLIT = false>
 __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t* s_st0, uint8_t* s_st1,
                                            uint8_t* s_st2, uint8_t* s_st3, int& s_vover)
 {
@@ -389,8 +391,9 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
     const int nrb = (R + kDmaRows - 1) / kDmaRows;
     // a prefill split over its keys deals piece p of every group after piece p - 1 of all of them, so that the pieces
     // of one group spread over the XCDs where the groups are fewer
+    static_assert(!(PFX && SPLIT), "prefix partials have chunks of their own");
     const int groups0 = PFX ? Hkv * a.pfx_chunks : a.batch * Hkv;
-    const int nsp = PFX || a.n_split < 1 ? 1 : a.n_split;
+    const int nsp = SPLIT ? a.n_split : 1;
     const int groups = groups0 * nsp;
 #if FFKV_PREFILL_XCD
     const int wg = wg_index;
@@ -484,7 +487,7 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
         pg_hi = static_cast<int>((kw + kBlockSize - 1) / kBlockSize);
     }
     int64_t part = -1;  // slot of this piece's partials, or -1: the workgroup has all the keys and writes the output
-    if (!PFX && nsp > 1)
+    if constexpr (SPLIT)
     {
         int64_t row_keys = ctx + S;
         row_keys = row_keys > L ? L : (row_keys < 0 ? 0 : row_keys);
@@ -1289,7 +1292,7 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
                 }
             }
         }
-        else if (part >= 0)
+        else if (SPLIT && part >= 0)
         {
             // partial of the row block's piece: the accumulators as the lanes hold them (whole 1 KiB stores), one
             // (max in the log2 domain, denominator) per query row
@@ -1317,7 +1320,7 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
     }
 }
 
-template <int QT, int D, int CT, bool PFX, int RG>
+template <int QT, int D, int CT, bool PFX, int RG, bool SPLIT>
 __global__ __launch_bounds__(512 / RG)
 __attribute__((amdgpu_waves_per_eu(RG == 2 ? (D == 256 ? 1 : 2) : (D <= 128 ? (CT == I8 ? 3 : 4) : 1))))
 void paged_prefill_dma(PrefillArgs a)
@@ -1328,7 +1331,7 @@ void paged_prefill_dma(PrefillArgs a)
     __shared__ __align__(16) uint8_t s_st2[L::S2];
     __shared__ __align__(16) uint8_t s_st3[L::S3];
     __shared__ int s_vover;
-    prefill_wg<QT, D, CT, PFX, RG>(a, static_cast<int>(blockIdx.x), s_st0, s_st1, s_st2, s_st3, s_vover);
+    prefill_wg<QT, D, CT, PFX, RG, SPLIT>(a, static_cast<int>(blockIdx.x), s_st0, s_st1, s_st2, s_st3, s_vover);
 }
 
 #ifndef FFKV_DEVICE_BODIES_ONLY
@@ -1412,7 +1415,7 @@ PrefillKernel prefill_kernel_d(int head_dim)
 {
     auto k = []<int D, int RG>()
     {
-        return PrefillKernel{reinterpret_cast<const void*>(paged_prefill_dma<QT, D, CT, false, RG>), 512 / RG,
+        return PrefillKernel{reinterpret_cast<const void*>(paged_prefill_dma<QT, D, CT, false, RG, true>), 512 / RG,
                              DmaCfg<D, kElemBytes<CT>, CT == I8, 8 / RG, false>::KP * kBlockSize};
     };
     if (head_dim == 64) return k.template operator()<64, FFKV_PREFILL_RG>();
@@ -1462,12 +1465,12 @@ hipError_t launch_prefill_merge_q(const PrefillArgs& a, hipStream_t stream)
     return hipGetLastError();
 }
 
-template <int CT, int QT, bool PFX>
+template <int CT, int QT, bool PFX, bool SPLIT>
 hipError_t launch_pfd_d(const PrefillArgs& a, hipStream_t stream)
 {
     const int64_t rows = PFX ? static_cast<int64_t>(a.batch) * a.group : static_cast<int64_t>(a.seq_len) * a.group;
     const int64_t groups = PFX ? static_cast<int64_t>(a.num_kv_heads) * a.pfx_chunks
-                               : static_cast<int64_t>(a.batch) * a.num_kv_heads * (a.n_split > 1 ? a.n_split : 1);
+                               : static_cast<int64_t>(a.batch) * a.num_kv_heads * (SPLIT ? a.n_split : 1);
     const int64_t nrb = (rows + kDmaRows - 1) / kDmaRows;
 #if FFKV_PREFILL_XCD
     const int64_t wgs = (groups + kXcds - 1) / kXcds * kXcds * nrb;
@@ -1483,36 +1486,36 @@ hipError_t launch_pfd_d(const PrefillArgs& a, hipStream_t stream)
     switch (a.head_dim)
     {
         case 64:
-            hipLaunchKernelGGL((paged_prefill_dma<QT, 64, CT, PFX, RG>), grid, dim3(512 / RG), 0, stream, a);
+            hipLaunchKernelGGL((paged_prefill_dma<QT, 64, CT, PFX, RG, SPLIT>), grid, dim3(512 / RG), 0, stream, a);
             break;
         case 128:
-            hipLaunchKernelGGL((paged_prefill_dma<QT, 128, CT, PFX, RG>), grid, dim3(512 / RG), 0, stream, a);
+            hipLaunchKernelGGL((paged_prefill_dma<QT, 128, CT, PFX, RG, SPLIT>), grid, dim3(512 / RG), 0, stream, a);
             break;
         default:
         {
             constexpr int RG256 = PFX ? 1 : FFKV_PREFILL_RG256;
-            hipLaunchKernelGGL((paged_prefill_dma<QT, 256, CT, PFX, RG256>), grid, dim3(512 / RG256), 0, stream, a);
+            hipLaunchKernelGGL((paged_prefill_dma<QT, 256, CT, PFX, RG256, SPLIT>), grid, dim3(512 / RG256), 0, stream, a);
             break;
         }
     }
     return hipGetLastError();
 }
 
-template <int CT, bool PFX>
+template <int CT, bool PFX, bool SPLIT>
 hipError_t launch_pfd_q(const PrefillArgs& a, hipStream_t stream)
 {
     switch (a.qo_dtype)
     {
         case F32:
-            return launch_pfd_d<CT, F32, PFX>(a, stream);
+            return launch_pfd_d<CT, F32, PFX, SPLIT>(a, stream);
         case F16:
-            return launch_pfd_d<CT, F16, PFX>(a, stream);
+            return launch_pfd_d<CT, F16, PFX, SPLIT>(a, stream);
         default:
-            return launch_pfd_d<CT, BF16, PFX>(a, stream);
+            return launch_pfd_d<CT, BF16, PFX, SPLIT>(a, stream);
     }
 }
 
-template <bool PFX>
+template <bool PFX, bool SPLIT>
 hipError_t launch_pfd(const PrefillArgs& a, hipStream_t stream)
 {
     // 8-bit caches read their scales in every workgroup (int8 per token, fp8 per head)
@@ -1521,13 +1524,13 @@ hipError_t launch_pfd(const PrefillArgs& a, hipStream_t stream)
     switch (a.cache_dtype)
     {
         case F16:
-            return launch_pfd_q<F16, PFX>(a, stream);
+            return launch_pfd_q<F16, PFX, SPLIT>(a, stream);
         case BF16:
-            return launch_pfd_q<BF16, PFX>(a, stream);
+            return launch_pfd_q<BF16, PFX, SPLIT>(a, stream);
         case I8:
-            return launch_pfd_q<I8, PFX>(a, stream);
+            return launch_pfd_q<I8, PFX, SPLIT>(a, stream);
         default:
-            return launch_pfd_q<FP8, PFX>(a, stream);
+            return launch_pfd_q<FP8, PFX, SPLIT>(a, stream);
     }
 }
 
@@ -1581,14 +1584,15 @@ PrefillSplitLayout prefill_split_layout(const PrefillArgs& a)
 
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t stream)
 {
-    const hipError_t e = launch_pfd<false>(a, stream);
-    if (e != hipSuccess || a.n_split <= 1) return e;
+    if (a.n_split <= 1) return launch_pfd<false, false>(a, stream);
+    const hipError_t e = launch_pfd<false, true>(a, stream);
+    if (e != hipSuccess) return e;
     if (a.qo_dtype == F32) return launch_prefill_merge_q<F32>(a, stream);
     if (a.qo_dtype == F16) return launch_prefill_merge_q<F16>(a, stream);
     return launch_prefill_merge_q<BF16>(a, stream);
 }
 
-hipError_t launch_prefix_partials(const PrefillArgs& a, hipStream_t stream) { return launch_pfd<true>(a, stream); }
+hipError_t launch_prefix_partials(const PrefillArgs& a, hipStream_t stream) { return launch_pfd<true, false>(a, stream); }
 
 #endif  // FFKV_DEVICE_BODIES_ONLY
 
