@@ -402,7 +402,8 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
     const int rb = nrb - 1 - k_in_xcd % nrb;
     int       grp = (k_in_xcd / nrb) * kXcds + xcd;
     const int g8 = (groups + kXcds - 1) / kXcds;  // group slots of this XCD: groups j * kXcds + xcd, j < g8
-    if (!PFX && a.paged && g8 <= 64 && g8 > 1)
+    // (one row has one length: its groups keep their order, and the ranking of up to 64 of a split call's cost 0.2 to 1.5 us)
+    if (!PFX && a.paged && a.batch > 1 && g8 <= 64 && g8 > 1)
     {
         // The XCD's groups by decreasing cached length (ties by index): lane j ranks group j * kXcds + xcd, and
         // the workgroup takes the group ranked k_in_xcd / nrb.  Absent groups (past `groups`) rank last.
@@ -1542,14 +1543,15 @@ hipError_t launch_pfd(const PrefillArgs& a, hipStream_t stream)
 // that call, of which 7.5 us are the merge; 4 pieces took 75 us, 16 took 61, 32 took 69).  A piece's partials (64 KiB at
 // head_dim 128) and the merge cost about as much as 5 steps, and at two pieces a split only puts a second workgroup on
 // each CU, so short calls stay whole.  Whole -> split in us, 32 / 8 heads of 128 dims, by the steps of the last block:
-//   8 pieces (one request's 256 tokens)   8: 20.4 -> 21.5, 10: 23.4 -> 22.8, 12: 26.2 -> 23.5, 16: 32.6 -> 26.0
-//   32 pieces (64 tokens)                 8: 19.8 -> 18.7,  9: 21.3 -> 17.6, 12: 26.4 -> 19.5
-//   4 pieces (512 tokens; 3 x 160)       13: 28.6 -> 30.5, 14: 30.2 -> 30.6, 15: 31.2 -> 31.1, 16: 32.8 -> 31.7
+//   8 pieces (one request's 256 tokens)   8: 20.1 -> 21.0, 11: 24.5 -> 22.4, 12: 25.9 -> 22.9, 20: 38.7 -> 28.8
+//   32 pieces (64 tokens)                 8: 19.5 -> 16.9,  9: 21.2 -> 15.9, 17: 34.1 -> 18.7
+//   4 pieces (3 x 160; 512 tokens)       13: 28.9 -> 30.4, 14: 30.3 -> 30.5, 15: 31.4 -> 30.3, 16: 32.5 -> 31.0
 //   2 pieces (3 x 256; 8 x 128)          18: 38.5 -> 41.0, 20: 40.4 -> 41.4, 22: 43.8 -> 43.2, 25: 48.8 -> 46.6
 // The host knows only the bound on a row (max_context_len, or the table's width): a call whose bound is below the point
 // where a split gains is not planned for one.  A planned call pays for the merge's launch whatever its rows turn out to
-// be (2.2 to 3.4 us: a first chunk of 256 tokens behind a wide table 13.3 -> 15.8), so its rows are split from a little
-// earlier on (split_from), where that costs no more than the empty merge.
+// be (1.9 us: a first chunk of 256 tokens behind a wide table 12.9 -> 14.8), so its rows are split from a little earlier
+// on (split_from), where that costs no more than the empty merge.  A caller that gives max_context_len pays it only where
+// rows may be long.
 void prefill_plan(PrefillArgs& a)
 {
     a.n_split = 1;
