@@ -87,13 +87,13 @@ hipError_t launch_row1(const DecodeArgs& a, hipStream_t stream)
 // alike), so a workgroup takes 6 us and 11 us per 512 KiB of its row; the split decode takes 11 to 14 us for the smallest
 // batches and 20 to 30 us from 16 rows on.  The row's length is not known here, only its bound (max_context_len or the
 // table's width), so the rule holds for rows as long as that.  Whole calls (append included), split -> row, us:
-//   up to 256 KiB of K and V per (row, KV head), up to 512 workgroups: 4 rows of 17 to 255 tokens at 16/8 heads 12.1 ->
-//   8.4; 1 row of 500 tokens 11.3 -> 10.7, 8 rows 13.8 -> 11.7, 16 rows 16.6 -> 12.0, 64 rows of 100 to 500 24.8 -> 23.4;
-//   32 rows of 500 to 1000 tokens of 64 dims 19.7 -> 14.5, on int8 pages of 128 dims 27.7 -> 22.2
-//   up to 512 KiB, 128 to 256 workgroups: 16 rows of 500 to 1000 tokens 20.2 -> 18.3, 32 rows 29.7 -> 22.4, 32 rows of 200
-//   to 400 tokens of 256 dims 30.3 -> 21.3
-// Beyond that the split is ahead: 1 row of 1000 tokens 13.3 against 16.0, 8 rows of 200 to 800 14.2 against 15.2, 48 rows of
-// 100 to 1000 28.8 against 30.0 (more workgroups than CUs), 128 rows of 50 to 250 26.2 against 30.0.
+//   up to 256 KiB of K and V per (row, KV head), up to 512 workgroups: 4 rows of 17 to 255 tokens at 16/8 heads 9.3 -> 6.9;
+//   at 32/8 heads 1 row of 500 tokens 9.7 -> 9.2, 8 rows of 100 to 500 10.5 -> 9.4, 16 rows 13.3 -> 9.8, 64 rows 23.1 ->
+//   21.3; 32 rows of 500 to 1000 tokens of 64 dims 17.6 -> 11.6, on int8 pages of 128 dims 25.9 -> 21.4
+//   up to 512 KiB, 128 to 256 workgroups: 16 rows of 500 to 1000 tokens 16.8 -> 16.1, 32 rows 25.2 -> 21.1, 32 rows of 200
+//   to 400 tokens of 256 dims 27.3 -> 19.6
+// Beyond that the split is ahead: 1 row of 1000 tokens 10.6 against 13.4, 8 rows of 200 to 800 11.7 against 12.9, 48 rows of
+// 100 to 1000 26.9 against 27.3 (more workgroups than CUs), 128 rows of 50 to 250 24.3 against 26.5.
 bool decode_use_row(const DecodeArgs& a)
 {
     const int64_t wgs = static_cast<int64_t>(a.batch) * a.num_kv_heads * ((a.group + 15) / 16);

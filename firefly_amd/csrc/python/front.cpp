@@ -4,8 +4,8 @@
 // once per layer.  Through ctypes a call cost 6 to 8 us before anything was launched: about 20 argument conversions,
 // and a Python call for every pointer, shape and dtype.  Here the wrappers of firefly_amd/__init__.py hand their
 // tensors over as they are, and shapes, dtypes, pointers and the current stream are read natively: 1 to 2 us.  The fused
-// append + decode of 4 rows of up to 255 tokens (16/8 heads), two launches: 12.5 -> 9.7 us in a row, where the GPU now
-// sets the pace, and 38 -> 25 us for a first call that is waited for.
+// append + decode of 4 rows of up to 255 tokens (16/8 heads), one launch: 10.1 -> 6.9 us in a row, where the GPU now sets
+// the pace, and 24.2 -> 19.1 us for a call that is waited for.
 // The library is the one firefly_amd loaded: bind() gets the addresses of its functions, so nothing is linked here.
 // Only CPython's own API is used; tensors are read through their attributes (shape, dtype, data_ptr(), nbytes).
 #define PY_SSIZE_T_CLEAN
@@ -120,19 +120,27 @@ struct Reader
         ok = false;
         return 0;
     }
-    int integer(PyObject* o)
+    int integer(PyObject* o)  // a Python int: nothing that merely converts to one (a device tensor would synchronize)
     {
         if (!ok) return 0;
+        if (!PyLong_Check(o))
+        {
+            PyErr_Format(PyExc_TypeError, "an int is required, not %.100s", Py_TYPE(o)->tp_name);
+            ok = false;
+            return 0;
+        }
         const long long v = PyLong_AsLongLong(o);
         if (v == -1 && PyErr_Occurred()) ok = false;
         return static_cast<int>(v);
     }
     int blocks(PyObject* num_blocks, PyObject* cache) { return num_blocks == Py_None ? dim(cache, 0) : integer(num_blocks); }
-    float real(PyObject* o)
+    float real(PyObject* o)  // whatever float() takes
     {
         if (!ok) return 0.0f;
-        const double v = PyFloat_AsDouble(o);
-        if (v == -1.0 && PyErr_Occurred()) ok = false;
+        PyObject*    f = PyNumber_Float(o);
+        const double v = f ? PyFloat_AS_DOUBLE(f) : 0.0;
+        Py_XDECREF(f);
+        if (f == nullptr) ok = false;
         return static_cast<float>(v);
     }
     size_t nbytes(PyObject* t)

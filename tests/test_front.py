@@ -4,6 +4,7 @@ there is no current one."""
 
 import threading
 
+import numpy as np
 import pytest
 import torch
 
@@ -67,6 +68,24 @@ def test_argument_errors(ff):
         ff.append_kv_cache(k, v, kc, vc, bt, cx, num_blocks="4", stream=0)
     with pytest.raises((TypeError, ValueError)):
         ff.append_kv_cache(k, v, kc, vc, bt, cx, stream="x")
+
+
+@pytest.mark.parametrize("n", [4.0, torch.tensor(4), np.int64(4)])
+def test_integers_are_ints(ff, n):
+    """num_blocks and max_context_len take a Python int (or a bool), as ctypes' c_int does, and no value that converts to
+    one; scale and theta take what float() takes."""
+    k, v, kc, vc, bt, cx = _args()
+    q = torch.zeros(0, 1, 2 * HKV, D, dtype=torch.bfloat16)
+    with pytest.raises(TypeError):
+        ff.append_kv_cache(k, v, kc, vc, bt, cx, num_blocks=n, stream=0)
+    with pytest.raises(TypeError):
+        ff.paged_attention(q, kc, vc, bt, cx, max_context_len=n, stream=0)
+    ff.append_kv_cache(k, v, kc, vc, bt, cx, num_blocks=True, stream=0)
+    ff.paged_attention(q, kc, vc, bt, cx, scale=n, stream=0)
+    ff.paged_attention(q, kc, vc, bt, cx, scale="0.5", stream=0)
+    ff.apply_rope(q, k, cx, theta=n, stream=0)
+    with pytest.raises(ValueError):
+        ff.paged_attention(q, kc, vc, bt, cx, scale="x", stream=0)
 
 
 def test_threads(ff):
