@@ -1,9 +1,10 @@
 """firefly_amd - MI355X (gfx950) paged KV-cache path for Firefly.
 
 The product is the shared library ``firefly_amd/libffkv.so`` (C ABI in ``include/ffkv.h``; C++ API in
-``include/firefly/``).  This module loads it with ctypes and offers thin wrappers that take torch tensors, so
-tests and benchmarks can drive the C ABI with device memory torch allocated.  There is no CPU fallback: if the
-library is missing or fails to load, importing this package raises.
+``include/firefly/``).  This module loads it and offers thin wrappers that take torch tensors, so programs, tests
+and benchmarks can drive the C ABI with device memory torch allocated: the calls of a step go through ``_front.so``
+(csrc/python/front.cpp, built with the library), sizes and the like through ctypes.  There is no CPU fallback: if
+either is missing or fails to load, importing this package raises.
 """
 
 from __future__ import annotations
@@ -180,8 +181,9 @@ def paged_prefill(q, k_cache, v_cache, block_table, context_lens, out=None, k_sc
 
 def _prefill_scratch(n: int, q, stream):
     """Scratch of ``n`` bytes for one call on ``stream`` (None: the current one), from torch's allocator and belonging
-    to that stream, so that it can be reused once the call's work on the stream is done.  None while the stream is
-    being captured (a capture allocates nothing here; the call then runs unsplit)."""
+    to that stream, so that it can be reused once the call's work on the stream is done.  None, where the call
+    runs unsplit, while the stream is being captured (a capture allocates nothing here) and where there is no memory
+    for it."""
     import torch
 
     if stream is not None:
@@ -191,7 +193,10 @@ def _prefill_scratch(n: int, q, stream):
             return _prefill_scratch(n, q, None)
     if torch.cuda.is_current_stream_capturing():
         return None
-    return torch.empty(n, dtype=torch.uint8, device=q.device)
+    try:
+        return torch.empty(n, dtype=torch.uint8, device=q.device)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def apply_rope(q, k, context_lens=None, theta: float = 1e6, stream=None) -> None:

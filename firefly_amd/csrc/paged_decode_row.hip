@@ -84,8 +84,8 @@ hipError_t launch_row1(const DecodeArgs& a, hipStream_t stream)
 }  // namespace
 
 // One CU draws about 47 GB/s of pages whatever its waves keep in flight (8 or 12 waves, two or three pages each, measured
-// alike), so a workgroup takes 6 us and 11 us per 512 KiB of its row; the split decode takes 11 to 14 us for the smallest
-// batches and 20 to 30 us from 16 rows on.  The row's length is not known here, only its bound (max_context_len or the
+// alike), so a workgroup takes 6 us and 11 us per 512 KiB of its row; the split decode takes 9 to 12 us for the smallest
+// batches and 13 to 27 us from 16 rows on.  The row's length is not known here, only its bound (max_context_len or the
 // table's width), so the rule holds for rows as long as that.  Whole calls (append included), split -> row, us:
 //   up to 256 KiB of K and V per (row, KV head), up to 512 workgroups: 4 rows of 17 to 255 tokens at 16/8 heads 9.3 -> 6.9;
 //   at 32/8 heads 1 row of 500 tokens 9.7 -> 9.2, 8 rows of 100 to 500 10.5 -> 9.4, 16 rows 13.3 -> 9.8, 64 rows 23.1 ->

@@ -88,6 +88,20 @@ def test_integers_are_ints(ff, n):
         ff.paged_attention(q, kc, vc, bt, cx, scale="x", stream=0)
 
 
+def test_prefill_scratch_without_memory(ff, monkeypatch):
+    """No memory for a split prefill's scratch: the call runs unsplit, as it does while its stream is captured."""
+    def full(*a, **kw):
+        raise torch.OutOfMemoryError("full")
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    assert ff._prefill_scratch(64, torch.empty(1), None).numel() == 64
+    monkeypatch.setattr(torch, "empty", full)
+    assert ff._prefill_scratch(64, torch.zeros(1), None) is None
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: pytest.fail("allocated under capture"))
+    assert ff._prefill_scratch(64, torch.zeros(1), None) is None
+
+
 def test_threads(ff):
     """The interpreter lock is given up around the library's call; its error message is the calling thread's."""
     k, v, kc, vc, bt, cx = _args(B=1)

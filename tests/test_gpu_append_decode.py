@@ -102,7 +102,8 @@ def test_head_shapes(ff, gpu, D, G):
 @pytest.mark.parametrize("act,kv", [("f32", "bf16"), ("bf16", "i8"), ("bf16", "fp8"), ("f32", "f32"),
                                     ("f16", "f16")])
 def test_two_launch_forms(ff, gpu, act, kv):
-    """Source dtype other than the cache's, quantized and fp32 caches: append kernel then decode."""
+    """Source dtype other than the cache's, quantized and fp32 caches: append kernel then decode (and f16 in its own
+    dtype, in one launch)."""
     rng = np.random.default_rng(75)
     c = cases.make_case(75, 7, 32, 8, 128, rng.integers(0, 900, size=7), act=act, kv=kv)
     _run(ff, gpu, c)

@@ -1,7 +1,6 @@
-"""The decode step on quantized caches in one call, where the decode itself quantizes the new token into its page before
-it loads that page: pages, codes and int8 scales byte for byte as the append kernel writes them, outputs within the bar
-of the CPU checker.  Both launches that do it (one workgroup per row behind the narrow table, the split behind one padded
-with -1), and the append launch beside them where the bound on the call's bytes passes 1 GiB.
+"""The decode step on quantized caches in one call: pages, codes and int8 scales byte for byte as the append kernel
+writes them, outputs within the bar of the CPU checker.  Both forms of the decode after the append launch: one workgroup
+per row behind the narrow table, the split behind one padded with -1.
 """
 
 import numpy as np
@@ -23,8 +22,8 @@ def _wide(c, blocks):
 @pytest.mark.parametrize("D,G,act", [(64, 1, "bf16"), (64, 20, "f16"), (80, 4, "bf16"), (96, 7, "f16"), (112, 2, "bf16"),
                                      (128, 4, "bf16"), (128, 17, "f32"), (256, 8, "bf16")])
 def test_forms(ff, gpu, kv, D, G, act):
-    """Every head_dim and source type; a group of 17 or 20 has two blocks of query heads, which both write the token;
-    odd KV-head counts put two heads of a token on one cache line."""
+    """Every head_dim and source type; a group of 17 or 20 has two blocks of query heads; odd KV-head counts put two heads
+    of a token on one cache line."""
     if (act, kv) == ("f16", "fp8") and D == 96:
         act = "f32"
     c = cases.make_case(6000 + D + G, 6, 3 * G, 3, D, [0, 15, 16, 31, 200, 333], act=act, kv=kv)
@@ -37,15 +36,14 @@ def test_many_rows(ff, gpu, kv):
     """Several windows of rows; many rows' ends in one wave's share of pages; 8 KV heads in workgroups of 4 or 8."""
     rng = np.random.default_rng(61)
     c = cases.make_case(6100, 150, 16, 8, 128, rng.integers(0, 300, size=150), act="bf16", kv=kv)
-    for table in (c.block_table, _wide(c, 100), _wide(c, 3500)):  # row or split, split, append launch
+    for table in (c.block_table, _wide(c, 100), _wide(c, 3500)):  # row or split, split, split over a bound of more than 1 GiB
         _run(ff, gpu, c, table=table)
 
 
 @pytest.mark.parametrize("kv", ["i8", "fp8"])
 @pytest.mark.parametrize("cap", [16, 500, 1000])
 def test_truncated(ff, gpu, kv, cap):
-    """Rows cut short by max_context_len: their tokens are quantized into their slots by the first wave (the row's own in
-    the one-launch kernel) without being attended."""
+    """Rows cut short by max_context_len: their tokens are quantized into their slots without being attended."""
     rng = np.random.default_rng(62)
     c = cases.make_case(6200 + cap, 70, 16, 4, 128, rng.integers(200, 900, size=70), act="bf16", kv=kv)
     _run(ff, gpu, c, max_context_len=cap)

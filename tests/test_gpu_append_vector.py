@@ -1,6 +1,6 @@
-"""The decode step in one call on the vector kernel: on fp32 pages the chunk that holds a row's last token takes it from
-k / v, attends it and writes it to its slot; 16-bit pages of head dims the matrix cores do not take run the append kernel
-first.  Pages byte for byte as the append kernel writes them, outputs within the bar of the CPU checker."""
+"""The decode step in one call on the vector kernel (fp32 pages, and head dims that the matrix cores do not take): the
+append kernel, then the decode.  Pages byte for byte as the append kernel writes them, outputs within the bar of the CPU
+checker."""
 
 import numpy as np
 import pytest
@@ -41,3 +41,11 @@ def test_other_source_types(ff, gpu, act, kv):
     rng = np.random.default_rng(73)
     c = cases.make_case(7300, 5, 16, 4, 128, rng.integers(0, 600, size=5), act=act, kv=kv)
     _run(ff, gpu, c)
+
+
+@pytest.mark.parametrize("D,act,kv", [(88, "bf16", "i8"), (40, "bf16", "fp8"), (88, "f32", "fp8")])
+@pytest.mark.parametrize("cap", [0, 16, 300])
+def test_quantized(ff, gpu, D, act, kv, cap):
+    """8-bit pages of the vector kernel's head dims, with and without rows cut short by max_context_len."""
+    c = cases.make_case(7400 + D, 6, 8, 2, D, [15, 16, 299, 300, 301, 700], act=act, kv=kv)
+    _run(ff, gpu, c, max_context_len=cap)

@@ -166,6 +166,61 @@ def test_cxx_api_chunked_prefill_over_cached_prefix(shim, gpu):
 
 
 @pytest.mark.gpu
+def test_cxx_api_split_prefill(ff, shim, gpu):
+    """A chunk over a long prefix, which the library splits over its keys with the workspace that kernels::attention keeps
+    per stream: eager on two streams in turn (one of them with its workspace released between), and captured over the
+    workspace of an eager call, its replays between other calls; all the same bits, within the bar of the checker."""
+    import torch
+
+    import gpu_util as gu
+
+    c = cases.make_case(93, 1, 16, 4, 128, [2100], act="bf16", S=20)
+    rng = np.random.default_rng(94)
+    qn = cases.encode(rng.standard_normal((c.B, c.S, c.Hq, c.D), dtype=np.float32), c.act)
+    assert ff.lib.ffkv_prefill_workspace_bytes(c.act, c.kv, c.B, c.S, c.Hq, c.Hkv, c.D, 1, c.max_blocks, 0) > 0
+    dq, kn, vn = gu.to_dev(qn, c.act, gpu), gu.to_dev(c.k_new, c.act, gpu), gu.to_dev(c.v_new, c.act, gpu)
+    dk, dv = gu.to_dev(c.k_pool, c.kv, gpu), gu.to_dev(c.v_pool, c.kv, gpu)
+    bt, ctx = torch.from_numpy(c.block_table).to(gpu), torch.from_numpy(c.ctx).to(gpu)
+
+    def call(out, stream):
+        rc = shim.kas_paged_prefill(dq.data_ptr(), kn.data_ptr(), vn.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                                    out.data_ptr(), bt.data_ptr(), ctx.data_ptr(), c.B, c.S, c.Hq, c.Hkv, c.D,
+                                    c.num_blocks, c.max_blocks, c.act, c.kv, stream.cuda_stream)
+        assert rc == 0, shim.kas_last_error()
+
+    new = lambda: torch.full((c.B, c.S, c.Hq * c.D), float("nan"), dtype=dq.dtype, device=gpu)
+    sides = [torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = [new() for _ in range(6)]
+    torch.cuda.synchronize()
+    for i, out in enumerate(outs):
+        call(out, sides[i % 2])
+        if i == 3:
+            assert shim.kas_release_workspace(sides[1].cuda_stream) == 0, shim.kas_last_error()
+    torch.cuda.synchronize()
+    rk, rv = c.k_pool.copy(), c.v_pool.copy()
+    O.append(c.k_new, c.v_new, c.act, rk, rv, c.kv, c.block_table, c.ctx)
+    ref = O.paged_prefill_f64(qn, c.act, rk, rv, c.kv, c.block_table, c.ctx)
+    assert _excess_bf16(outs[0].float().cpu().numpy().reshape(ref.shape), ref) <= 2e-3
+    assert all(torch.equal(o, outs[0]) for o in outs)
+    whole = torch.empty_like(outs[0])  # (the unsplit call: other bits, so the calls above are split)
+    ff.check(ff.lib.ffkv_paged_prefill(dq.data_ptr(), whole.data_ptr(), c.act, dk.data_ptr(), dv.data_ptr(), c.kv, None,
+                                       None, bt.data_ptr(), ctx.data_ptr(), c.B, c.S, c.Hq, c.Hkv, c.D, 16, c.max_blocks,
+                                       c.num_blocks, 0, 0.0, ff._stream(None)))
+    assert not torch.equal(whole, outs[0])
+    captured = new()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=sides[0]):
+        call(captured, sides[0])
+    for _ in range(3):
+        captured.zero_()
+        g.replay()
+        call(outs[1], torch.cuda.current_stream())
+        torch.cuda.synchronize()
+        assert torch.equal(captured, outs[0]) and torch.equal(outs[1], outs[0])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("act,kv", [("bf16", "bf16"), ("f16", "i8"), ("bf16", "fp8")])
 @pytest.mark.parametrize("fused", [1, 0])
 def test_cxx_api_rope_then_append(shim, gpu, act, kv, fused):
