@@ -87,8 +87,8 @@ struct PrefillArgs
     float*         ws_acc;
     // Prefill split over the keys (launch_prefill with n_split > 1): each block of 128 query rows takes up to n_split
     // pieces of its steps (the kernel's own number of keys), written as partials to the workspace and merged by a
-    // second kernel.  Rows whose last block has fewer than split_from steps stay whole; a piece has at least
-    // kPrefillSplitMin steps, and as many more as it takes for all the call's pieces to fill split_slots workgroups once.  n_split <= 1: no
+    // second kernel.  A call none of whose rows has split_from steps stays whole; a piece has at least kPrefillSplitMin
+    // steps, and as many more as it takes for all the call's pieces to fill split_slots workgroups once.  n_split <= 1: no
     // pieces, no workspace.
     int            n_split;
     int            split_slots;

@@ -259,27 +259,34 @@ __device__ __forceinline__ void wait_vm()
     __builtin_amdgcn_s_waitcnt(VM | (0x7 << 4) | (0xF << 8));  // vmcnt(VM), expcnt and lgkmcnt not waited on
 }
 
-// Pieces that a block of `steps` steps, of a row whose last block has `row_steps`, is split into (a.n_split > 1):
-// as many as keep a piece at kPrefillSplitMin steps or more and all pieces of the call together at about split_slots
-// (the workgroups resident at once).  The call's steps are summed over its rows at the middle of their chunks.  A row is
-// split in all its blocks or in none: the blocks left whole beside split ones would last the longest.
+// Pieces that a block of `steps` steps, of a row whose last block has `row_steps`, is split into (a.n_split > 1), the same
+// in every workgroup of the call: none where no row of the call has split_from steps, else as many as keep a piece at
+// kPrefillSplitMin steps or more and all pieces of the call together at about split_slots (the workgroups resident at
+// once).  The call's steps are summed over its rows at the middle of their chunks.  All blocks of a call are split alike:
+// blocks left whole beside split ones would last the longest.
 template <int KP>
 __device__ __forceinline__ int split_pieces(const PrefillArgs& a, int steps, int row_steps, int nrb, int lane)
 {
     constexpr int KEYS = KP * kBlockSize;
-    if (row_steps < a.split_from) return 1;
+    if (a.batch == 1 && row_steps < a.split_from) return 1;
     int64_t total = 0;
+    bool    any = row_steps >= a.split_from;
     for (int b0 = 0; b0 < a.batch; b0 += 64)
     {
-        int st = 0;
+        int st = 0, last = 0;
         if (b0 + lane < a.batch)
         {
-            int64_t n = (a.paged ? static_cast<int64_t>(a.context_lens[b0 + lane]) : 0) + (a.seq_len + 1) / 2;
+            const int64_t ctx = a.paged ? static_cast<int64_t>(a.context_lens[b0 + lane]) : 0;
+            int64_t       n = ctx + (a.seq_len + 1) / 2;
             n = n < 0 ? 0 : (n > a.cap_tokens ? a.cap_tokens : n);
             st = static_cast<int>((n + KEYS - 1) / KEYS);
+            n = ctx + a.seq_len;
+            last = static_cast<int>((min(n, static_cast<int64_t>(a.cap_tokens)) + KEYS - 1) / KEYS);
         }
+        any = any || __any(last >= a.split_from);
         total += uniform(wave_sum(st));
     }
+    if (!any) return 1;
     total *= static_cast<int64_t>(a.num_kv_heads) * nrb;
     int64_t len = (total + a.split_slots - 1) / a.split_slots;
     len = len < kPrefillSplitMin ? kPrefillSplitMin : len;
@@ -401,22 +408,33 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
     const int k_in_xcd = wg / kXcds;
     const int rb = nrb - 1 - k_in_xcd % nrb;
     int       grp = (k_in_xcd / nrb) * kXcds + xcd;
-    const int g8 = (groups + kXcds - 1) / kXcds;  // group slots of this XCD: groups j * kXcds + xcd, j < g8
-    // (one row has one length: its groups keep their order, and the ranking of up to 64 of a split call's cost 0.2 to 1.5 us)
+    // group slots of this XCD: groups j * kXcds + xcd, j0 <= j < j0 + g8 (split: those of this workgroup's piece, the slots
+    // of a piece follow those of the piece before)
+    int g8 = (groups + kXcds - 1) / kXcds, j0 = 0, pc = 0;
+    if constexpr (SPLIT)
+    {
+        pc = grp / groups0;
+        j0 = (pc * groups0 - xcd + kXcds - 1) / kXcds;
+        g8 = ((pc + 1) * groups0 - xcd + kXcds - 1) / kXcds - j0;
+    }
+    // (one row has one length: its groups keep their order)
     if (!PFX && a.paged && a.batch > 1 && g8 <= 64 && g8 > 1)
     {
-        // The XCD's groups by decreasing cached length (ties by index): lane j ranks group j * kXcds + xcd, and
-        // the workgroup takes the group ranked k_in_xcd / nrb.  Absent groups (past `groups`) rank last.
-        const int gl = lane * kXcds + xcd;
-        const int wl = lane < g8 && gl < groups ? a.context_lens[(nsp == 1 ? gl : gl % groups0) / Hkv] : -2147483647 - 1;
+        // The XCD's groups by decreasing cached length (ties by index): lane j ranks group (j0 + j) * kXcds + xcd, and
+        // the workgroup takes the group ranked k_in_xcd / nrb - j0.  Absent groups (past `groups`) rank last.  (Pieces are
+        // not ranked beside each other: the first pieces of all groups go out first, to a CU each.  Ranked by length alone,
+        // the pieces past the end of a long row's lay between, and 4 x 33 tokens over 210 to 300 cached ones, which are not
+        // split, had their work on a quarter of the CUs: 24.0 us, 19.8 now, 17.0 unsplit.)
+        const int gl = (j0 + lane) * kXcds + xcd;
+        const int wl = lane < g8 && gl < groups ? a.context_lens[(gl - pc * groups0) / Hkv] : -2147483647 - 1;
         int       rank = 0;
         for (int m = 0; m < g8; ++m)
         {
             const int wm = __builtin_amdgcn_readlane(wl, m);
             rank += (wm > wl || (wm == wl && m < lane)) ? 1 : 0;
         }
-        const uint64_t hit = __ballot(lane < g8 && rank == k_in_xcd / nrb);
-        grp = hit != 0 ? (__ffsll(static_cast<long long>(hit)) - 1) * kXcds + xcd : groups;
+        const uint64_t hit = __ballot(lane < g8 && rank == k_in_xcd / nrb - j0);
+        grp = hit != 0 ? (j0 + __ffsll(static_cast<long long>(hit)) - 1) * kXcds + xcd : groups;
     }
     if (grp >= groups) return;  // padding of the grid to whole rounds of XCDs
 #else
@@ -1549,8 +1567,9 @@ hipError_t launch_pfd(const PrefillArgs& a, hipStream_t stream)
 //   2 pieces (3 x 256; 8 x 128)          18: 38.5 -> 41.0, 20: 40.4 -> 41.4, 22: 43.8 -> 43.2, 25: 48.8 -> 46.6
 // The host knows only the bound on a row (max_context_len, or the table's width): a call whose bound is below the point
 // where a split gains is not planned for one.  A planned call pays for the merge's launch whatever its rows turn out to
-// be (1.9 us: a first chunk of 256 tokens behind a wide table 12.9 -> 14.8), so its rows are split from a little earlier
-// on (split_from), where that costs no more than the empty merge.  A caller that gives max_context_len pays it only where
+// be (1.9 us: a first chunk of 256 tokens behind a wide table 12.9 -> 14.8; 2.5 to 3.2 for several rows, whose lengths
+// every workgroup reads), so it is split from a little earlier on (split_from), where that costs no more than the empty
+// merge.  A caller that gives max_context_len pays it only where
 // rows may be long.
 void prefill_plan(PrefillArgs& a)
 {

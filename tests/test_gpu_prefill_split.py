@@ -4,8 +4,8 @@ the unsplit call.
 Bar against the closed form as in test_gpu_prefill.py.  Split and unsplit differ by the order of fp32 sums and the
 reference maxima of P's rounding to 11 bits: both lie within the bar, so their difference is held to the sum of two.
 Each case says whether the library plans to split it (``ffkv_prefill_workspace_bytes``) at the edges of the rule on the
-bound of a row (12 steps of 64 keys at five pieces and more), or, behind a wide table, whether its rows are split at the
-edges of the rule on their own length (8 steps at eight pieces and more, 9 from five, 13 from three, 19 at two).
+bound of a row (12 steps of 64 keys at five pieces and more), or, behind a wide table, whether it is split at the edges of
+the rule on the longest row's own length (8 steps at eight pieces and more, 9 from five, 13 from three, 19 at two).
 """
 
 import numpy as np
@@ -111,20 +111,19 @@ def _pieces(ff, dev, c, qn, max_context_len=0):
 @pytest.mark.parametrize("B,Hq,Hkv,S,rule", [(1, 32, 8, 33, 8), (1, 32, 8, 256, 8), (1, 32, 8, 350, 9), (3, 32, 8, 160, 13),
                                              (3, 32, 8, 256, 19)])
 def test_wide_table(ff, gpu, B, Hq, Hkv, S, rule):
-    """32, 8, 5, 4 and 2 pieces planned for: rows one step short of the rule are whole, rows at it are split in every block
-    (all have more than four steps), and a bound below the rule's own plans nothing."""
+    """32, 8, 5, 4 and 2 pieces planned for: a call whose longest row is one step short of the rule is whole, one at it is
+    split in every block of more than four steps, also in a shorter row, and a bound below the rule's own plans nothing."""
     for steps in (rule - 1, rule):
-        ctx = [64 * steps - S] + [0] * (B - 1)
+        ctx = [0, 64 * 7 - S, 64 * steps - S][-B:] if B > 1 else [64 * steps - S]
         c, qn = _case(1000 + S + steps, B, Hq, Hkv, 128, ctx, S)
         # the pools hold the chunk's keys as well: nothing is appended
         ref = O.paged_prefill_f64(qn, c.act, c.k_pool, c.v_pool, c.kv, c.block_table, c.ctx)
         got, pieces = _pieces(ff, gpu, c, qn)
         _check(got.reshape(ref.shape), ref, c.act, 2e-3)
-        row0 = pieces.reshape(B, -1)[0]
-        assert (row0 > 1).any() == (steps == rule) and (pieces >= 1).all()
-        if steps == rule:
-            assert row0.min() >= 2
-        assert (pieces.reshape(B, -1)[1:] == 1).all()
+        split = pieces.reshape(B, -1) > 1
+        assert (pieces >= 1).all() and split[-1].all() == split.any() == (steps == rule)
+        assert B == 1 or split[-2].any() == split.any()
+        assert not split[:-2].any()
         got, pieces = _pieces(ff, gpu, c, qn, max_context_len=64 * 11)
         assert pieces is None
 
