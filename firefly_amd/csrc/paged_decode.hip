@@ -135,20 +135,23 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
         for (int i = 0; i < 8; ++i) acc[g][i] = 0.0f;
     }
 
-    // fp32 pages are read past the caches, unless a neighbouring row holds the chunk's first page too (a shared
-    // prefix, which the rows' workgroups then read from the caches).  32 rows of 512 to 4096 tokens at 32/8 heads take
-    // 128 us per call with plain loads and 114 (5.3 TB/s) with these, 120 rows over a 2048-token prefix 203 us with
-    // plain loads and 275 with these.  (Four token groups per trip gain another 1 % on the former and cost the latter
-    // 10 %: fewer waves fit.)
+    // fp32 pages are read past the caches, unless another row holds the chunk's first page too (a shared prefix, which the
+    // rows' workgroups then read from the caches).  32 rows of 512 to 4096 tokens at 32/8 heads take 128 us per call with
+    // plain loads and 113 with these, 120 rows over a 2048-token prefix 188 us with plain loads and 275 with these.  (Four
+    // token groups per trip gain another 1 % on the former and cost the latter 10 %: fewer waves fit.)  Any of the 256
+    // rows around this one counts, a thread each: rows over two or ten prefixes in turn, no two neighbours alike, took 296
+    // and 395 us where only the rows on either side were looked at, 194 and 357 now (all plain: 204 and 360).
     const int32_t* table = a.block_table + static_cast<int64_t>(b) * a.max_blocks;
     bool           once = CT == F32;
-    if (CT == F32 && begin < end)
+    if constexpr (CT == F32)
     {
-        const int own = table[begin >> 4];
-        for (int o = -1; o <= 1; o += 2)
-            if (b + o >= 0 && b + o < a.batch && table[(begin >> 4) + static_cast<int64_t>(o) * a.max_blocks] == own)
-                once = false;
-        once = __builtin_amdgcn_readfirstlane(once);
+        if (begin < end)  // uniform over the workgroup
+        {
+            const int r = max(0, min(b - 128, a.batch - 256)) + tid;
+            const bool other = r != b && r < a.batch &&
+                               a.block_table[static_cast<int64_t>(r) * a.max_blocks + (begin >> 4)] == table[begin >> 4];
+            once = __syncthreads_or(other) == 0;
+        }
     }
 
     // U consecutive token groups per loop trip: their table entries, then all their K / V loads, go out before

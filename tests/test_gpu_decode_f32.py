@@ -34,6 +34,17 @@ def test_decode_f32_shared_pages(ff, gpu, shared):
     _check(ff, gpu, c, 1e-4)
 
 
+@pytest.mark.parametrize("B", [6, 300])
+def test_decode_f32_prefixes_in_turn(ff, gpu, B):
+    """Rows over two prefixes in turn, so that no row shares pages with its neighbours, and rows of their own at the ends;
+    more rows than one workgroup looks at."""
+    ctx = [330 + 16 * (b % 3) for b in range(B)]
+    c = cases.make_case(730 + B, B, 4, 2, 64, ctx, act="f32", input_scale=1 / 8)
+    for b in range(3, B - 2):
+        c.block_table[b, :18] = c.block_table[1 + b % 2, :18]
+    _check(ff, gpu, c, 1e-4)
+
+
 @pytest.mark.parametrize("kv,tol", [("bf16", 2e-3), ("i8", 2e-2)])
 def test_vector_decode_merge(ff, gpu, kv, tol):
     """The same merge behind the vector kernel's other caches (head_dim 88)."""
