@@ -168,7 +168,9 @@ def paged_prefill(q, k_cache, v_cache, block_table, context_lens, out=None, k_sc
                   max_context_len: int = 0, scale: float = 0.0, num_blocks: int | None = None, stream=None):
     """Causal prefill attention (``ffkv_paged_prefill_ws``): ``q`` ``[B, S, Hq, D]`` over the paged cache (queries at
     ``context_lens[b] + t``), or, with ``block_table=None``, over contiguous ``k_cache``/``v_cache``
-    ``[B, S, Hkv, D]``.  Returns ``out`` ``[B, S, Hq * D]``."""
+    ``[B, S, Hkv, D]``.  Returns ``out`` ``[B, S, Hq * D]``.  Calls too small to fill the GPU are split over their keys
+    where the rows may be long; ``max_context_len`` (no row has more tokens, the chunk's included) says that they are
+    not, behind a wide table."""
     if out is None:
         import torch
 

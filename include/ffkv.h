@@ -224,8 +224,13 @@ FFKV_API int ffkv_paged_prefill(const void* q, void* out, int qo_dtype, const vo
  * ffkv_paged_prefill with scratch: a call with too few blocks of 128 query rows to fill the GPU (one request's chunk
  * over a long context, a short prompt) splits their keys into pieces that run side by side, whose partial results
  * live in `workspace` (ffkv_prefill_workspace_bytes; 16-byte aligned, any initial contents), and merges them.  Results
- * equal ffkv_paged_prefill's up to floating-point summation order.  ffkv_prefill_workspace_bytes is 0 where the call
- * would not be split; with workspace NULL, or fewer bytes than that, the call runs unsplit, as ffkv_paged_prefill.
+ * equal ffkv_paged_prefill's up to rounding: the sums take another order, and a piece rounds its attention weights to
+ * their 11 bits against a maximum of its own (together 1e-3 of the result in bf16, both equally far from the exact one);
+ * rows that are NaN are the same.  Equal calls give equal bits.
+ * The bound on a row (max_context_len, or the table's width) decides whether a split is planned:
+ * ffkv_prefill_workspace_bytes is 0 where it is not; with workspace NULL, or fewer bytes than that, the call runs unsplit,
+ * as ffkv_paged_prefill.  A planned call whose rows turn out too short is not split, but pays 2 to 3 us for the launch of
+ * a merge without work: give max_context_len where the rows' lengths are known and the table is wide.
  * Calls sharing one workspace must not overlap in time.  paged: whether the call has a block table.
  */
 FFKV_API size_t ffkv_prefill_workspace_bytes(int qo_dtype, int cache_dtype, int batch, int seq_len, int num_heads,
