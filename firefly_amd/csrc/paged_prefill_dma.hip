@@ -259,38 +259,64 @@ __device__ __forceinline__ void wait_vm()
     __builtin_amdgcn_s_waitcnt(VM | (0x7 << 4) | (0xF << 8));  // vmcnt(VM), expcnt and lgkmcnt not waited on
 }
 
-// Pieces that a block of `steps` steps, of a row whose last block has `row_steps`, is split into (a.n_split > 1), the same
-// in every workgroup of the call: none where no row of the call has split_from steps, else as many as keep a piece at
-// kPrefillSplitMin steps or more and all pieces of the call together at about split_slots (the workgroups resident at
-// once).  The call's steps are summed over its rows at the middle of their chunks.  All blocks of a call are split alike:
-// blocks left whole beside split ones would last the longest.
+// Lane of the r-th largest (from 0) of the keys of lanes 0 .. n - 1, the same in all lanes; keys from 0 to `bound`, equal ones
+// in the order of their lanes; -1 where r >= n.  A compare and a few scalar instructions per bit of the bound, where
+// ranking each lane against every other takes six vector instructions per lane (64 slots: 1 to 2 us of a call, 16 x 32
+// tokens over 490 to 700 cached ones 28.3 -> 26.5 us).
+__device__ __forceinline__ int nth_largest(uint32_t key, int bound, int n, int r, int lane)
+{
+    uint64_t in = n >= 64 ? ~uint64_t{0} : (uint64_t{1} << n) - 1;
+    for (int bit = 31 - __builtin_clz(bound | 1); bit >= 0; --bit)
+    {
+        const uint64_t set = __ballot((key >> bit & 1) != 0) & in;
+        const int      above = __popcll(set);
+        in = r < above ? set : in & ~set;
+        r -= r < above ? 0 : above;
+    }
+    const int      below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(in >> 32),
+                                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(in), 0));
+    const uint64_t hit = __ballot((in >> lane & 1) != 0 && below == r);
+    return __ffsll(static_cast<long long>(hit)) - 1;
+}
+
+// Steps of the query rows of a row with ctx cached tokens, up to the `n`-th of its chunk.
 template <int KP>
-__device__ __forceinline__ int split_pieces(const PrefillArgs& a, int steps, int row_steps, int nrb, int lane)
+__device__ __forceinline__ int row_steps(const PrefillArgs& a, int64_t ctx, int n)
 {
     constexpr int KEYS = KP * kBlockSize;
-    if (a.batch == 1 && row_steps < a.split_from) return 1;
+    const int64_t keys = min(max(ctx + n, int64_t{0}), static_cast<int64_t>(a.cap_tokens));
+    return static_cast<int>((keys + KEYS - 1) / KEYS);
+}
+
+// Steps of a piece of a call that may be split (a.n_split > 1), the same in every workgroup of the call: 0, the call stays
+// whole, where no row of it has split_from steps, else kPrefillSplitMin or as many more as leave all pieces of the call
+// together at about split_slots (the workgroups resident at once).  The call's steps are summed over its rows at the
+// middle of their chunks.  All blocks of a call are split alike: blocks left whole beside split ones would last the
+// longest.
+template <int KP>
+__device__ __forceinline__ int split_len(const PrefillArgs& a, int nrb, int lane)
+{
     int64_t total = 0;
-    bool    any = row_steps >= a.split_from;
+    bool    any = false;
     for (int b0 = 0; b0 < a.batch; b0 += 64)
     {
-        int st = 0, last = 0;
-        if (b0 + lane < a.batch)
-        {
-            const int64_t ctx = a.paged ? static_cast<int64_t>(a.context_lens[b0 + lane]) : 0;
-            int64_t       n = ctx + (a.seq_len + 1) / 2;
-            n = n < 0 ? 0 : (n > a.cap_tokens ? a.cap_tokens : n);
-            st = static_cast<int>((n + KEYS - 1) / KEYS);
-            n = ctx + a.seq_len;
-            last = static_cast<int>((min(n, static_cast<int64_t>(a.cap_tokens)) + KEYS - 1) / KEYS);
-        }
-        any = any || __any(last >= a.split_from);
-        total += uniform(wave_sum(st));
+        const bool    in = b0 + lane < a.batch;
+        const int64_t ctx = in && a.paged ? a.context_lens[b0 + lane] : 0;
+        any = any || __any(in && row_steps<KP>(a, ctx, a.seq_len) >= a.split_from);
+        if (!any && a.batch <= 64) return 0;
+        total += uniform(wave_sum(in ? row_steps<KP>(a, ctx, (a.seq_len + 1) / 2) : 0));
     }
-    if (!any) return 1;
-    total *= static_cast<int64_t>(a.num_kv_heads) * nrb;
-    int64_t len = (total + a.split_slots - 1) / a.split_slots;
-    len = len < kPrefillSplitMin ? kPrefillSplitMin : len;
-    const int np = static_cast<int>((steps + len - 1) / len);
+    if (!any) return 0;
+    total = total * a.num_kv_heads * nrb + a.split_slots - 1;
+    const int len = total >> 32 == 0 ? static_cast<int>(static_cast<uint32_t>(total) / static_cast<uint32_t>(a.split_slots))
+                                     : static_cast<int>(total / a.split_slots);
+    return max(len, kPrefillSplitMin);
+}
+
+// Pieces of a block of `steps` steps.
+__device__ __forceinline__ int split_pieces(const PrefillArgs& a, int steps, int len)
+{
+    const int np = len == 0 ? 1 : (steps + len - 1) / len;
     return np < 1 ? 1 : (np > a.n_split ? a.n_split : np);
 }
 
@@ -408,38 +434,63 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
     const int k_in_xcd = wg / kXcds;
     const int rb = nrb - 1 - k_in_xcd % nrb;
     int       grp = (k_in_xcd / nrb) * kXcds + xcd;
-    // group slots of this XCD: groups j * kXcds + xcd, j0 <= j < j0 + g8 (split: those of this workgroup's piece, the slots
-    // of a piece follow those of the piece before)
-    int g8 = (groups + kXcds - 1) / kXcds, j0 = 0, pc = 0;
+    int       len = 0;
     if constexpr (SPLIT)
     {
-        pc = grp / groups0;
-        j0 = (pc * groups0 - xcd + kXcds - 1) / kXcds;
-        g8 = ((pc + 1) * groups0 - xcd + kXcds - 1) / kXcds - j0;
+        // The pieces of an XCD's groups by decreasing steps, those without any last: the longest go out first and to a CU
+        // each.  Lane j holds group slot (j0 + j) * kXcds + xcd, of all pieces, or where those are more than the lanes of
+        // this workgroup's.  (Of equal rows, in the order of their pieces.  Piece after piece, the longest row first in
+        // each, the first and the second piece of the longest row met on a CU: 4 x 463 tokens over 900 to 7600 cached ones
+        // on int8 pages of 64 dims 131 us, 92 now.  By the rows' lengths alone, the idle pieces of long rows lay
+        // between: 4 x 33 tokens over 665 to 950 39 us, 25 now.)  A call that stays whole has at most half the blocks that
+        // are resident at once, in any order.
+        len = split_len<KP>(a, nrb, lane);
+        const int pc = grp / groups0;
+        if (len == 0 && pc > 0) return;
+        int g8 = (groups - xcd + kXcds - 1) / kXcds, j0 = 0;
+        if (g8 > 64)
+        {
+            j0 = (pc * groups0 - xcd + kXcds - 1) / kXcds;
+            g8 = ((pc + 1) * groups0 - xcd + kXcds - 1) / kXcds - j0;
+        }
+        if (len > 0 && a.paged && a.batch > 1 && g8 <= 64 && g8 > 1)
+        {
+            const int gl = (j0 + lane) * kXcds + xcd;
+            int       key = 0;
+            if (lane < g8 && gl < groups)
+            {
+                const int pl = gl / groups0;
+                const int st = row_steps<KP>(a, a.context_lens[(gl - pl * groups0) / Hkv], S);
+                const int np = split_pieces(a, st, len);
+                key = pl < np ? st / np : 0;
+            }
+            const int hit = nth_largest(static_cast<uint32_t>(key), max(len, row_steps<KP>(a, a.cap_tokens, 0) / nsp), g8,
+                                        k_in_xcd / nrb - j0, lane);
+            grp = hit >= 0 ? (j0 + hit) * kXcds + xcd : groups;
+        }
     }
     // (one row has one length: its groups keep their order)
-    if (!PFX && a.paged && a.batch > 1 && g8 <= 64 && g8 > 1)
+    const int g8 = (groups + kXcds - 1) / kXcds;  // group slots of this XCD: groups j * kXcds + xcd, j < g8
+    if (!PFX && !SPLIT && a.paged && a.batch > 1 && g8 <= 64 && g8 > 1)
     {
-        // The XCD's groups by decreasing cached length (ties by index): lane j ranks group (j0 + j) * kXcds + xcd, and
-        // the workgroup takes the group ranked k_in_xcd / nrb - j0.  Absent groups (past `groups`) rank last.  (Pieces are
-        // not ranked beside each other: the first pieces of all groups go out first, to a CU each.  Ranked by length alone,
-        // the pieces past the end of a long row's lay between, and 4 x 33 tokens over 210 to 300 cached ones, which are not
-        // split, had their work on a quarter of the CUs: 24.0 us, 19.8 now, 17.0 unsplit.)
-        const int gl = (j0 + lane) * kXcds + xcd;
-        const int wl = lane < g8 && gl < groups ? a.context_lens[(gl - pc * groups0) / Hkv] : -2147483647 - 1;
+        // The XCD's groups by decreasing cached length (ties by index): lane j ranks group j * kXcds + xcd, and
+        // the workgroup takes the group ranked k_in_xcd / nrb.  Absent groups (past `groups`) rank last.
+        const int gl = lane * kXcds + xcd;
+        const int wl = lane < g8 && gl < groups ? a.context_lens[gl / Hkv] : -2147483647 - 1;
         int       rank = 0;
         for (int m = 0; m < g8; ++m)
         {
             const int wm = __builtin_amdgcn_readlane(wl, m);
             rank += (wm > wl || (wm == wl && m < lane)) ? 1 : 0;
         }
-        const uint64_t hit = __ballot(lane < g8 && rank == k_in_xcd / nrb - j0);
-        grp = hit != 0 ? (j0 + __ffsll(static_cast<long long>(hit)) - 1) * kXcds + xcd : groups;
+        const uint64_t hit = __ballot(lane < g8 && rank == k_in_xcd / nrb);
+        grp = hit != 0 ? (__ffsll(static_cast<long long>(hit)) - 1) * kXcds + xcd : groups;
     }
     if (grp >= groups) return;  // padding of the grid to whole rounds of XCDs
 #else
     const int grp = wg_index / nrb;
     const int rb = wg_index % nrb;
+    const int len = SPLIT ? split_len<KP>(a, nrb, lane) : 0;
 #endif
     const int piece = nsp == 1 ? 0 : grp / groups0;
     const int grp0 = grp - piece * groups0;
@@ -508,10 +559,7 @@ __device__ __forceinline__ void prefill_wg(PrefillArgs a, int wg_index, uint8_t*
     int64_t part = -1;  // slot of this piece's partials, or -1: the workgroup has all the keys and writes the output
     if constexpr (SPLIT)
     {
-        int64_t row_keys = ctx + S;
-        row_keys = row_keys > L ? L : (row_keys < 0 ? 0 : row_keys);
-        const int row_steps = static_cast<int>((row_keys + KP * kBlockSize - 1) / (KP * kBlockSize));
-        const int np = split_pieces<KP>(a, (pg_hi + KP - 1) / KP, row_steps, nrb, lane);
+        const int np = split_pieces(a, (pg_hi + KP - 1) / KP, len);
         if (piece >= np) return;  // uniform over the workgroup
         const int64_t blk = static_cast<int64_t>(grp0) * nrb + rb;
         if (piece == 0 && tid == 0) a.ws_pieces[blk] = np;
@@ -1567,10 +1615,9 @@ hipError_t launch_pfd(const PrefillArgs& a, hipStream_t stream)
 //   2 pieces (3 x 256; 8 x 128)          18: 38.5 -> 41.0, 20: 40.4 -> 41.4, 22: 43.8 -> 43.2, 25: 48.8 -> 46.6
 // The host knows only the bound on a row (max_context_len, or the table's width): a call whose bound is below the point
 // where a split gains is not planned for one.  A planned call pays for the merge's launch whatever its rows turn out to
-// be (1.9 us: a first chunk of 256 tokens behind a wide table 12.9 -> 14.8; 2.5 to 3.2 for several rows, whose lengths
-// every workgroup reads), so it is split from a little earlier on (split_from), where that costs no more than the empty
-// merge.  A caller that gives max_context_len pays it only where
-// rows may be long.
+// be (1 to 2 us: a first chunk of 256 tokens behind a wide table 12.9 -> 14.8, 4 x 33 tokens over 210 to 300 with their
+// append 20.8 -> 21.8), so it is split from a little earlier on (split_from), where that costs no more than the empty
+// merge.  A caller that gives max_context_len pays it only where rows may be long.
 void prefill_plan(PrefillArgs& a)
 {
     a.n_split = 1;

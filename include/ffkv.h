@@ -229,7 +229,7 @@ FFKV_API int ffkv_paged_prefill(const void* q, void* out, int qo_dtype, const vo
  * rows that are NaN are the same.  Equal calls give equal bits.
  * The bound on a row (max_context_len, or the table's width) decides whether a split is planned:
  * ffkv_prefill_workspace_bytes is 0 where it is not; with workspace NULL, or fewer bytes than that, the call runs unsplit,
- * as ffkv_paged_prefill.  A planned call whose rows turn out too short is not split, but pays 2 to 3 us for the launch of
+ * as ffkv_paged_prefill.  A planned call whose rows turn out too short is not split, but pays 1 to 2 us for the launch of
  * a merge without work: give max_context_len where the rows' lengths are known and the table is wide.
  * Calls sharing one workspace must not overlap in time.  paged: whether the call has a block table.
  */

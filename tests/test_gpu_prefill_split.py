@@ -128,6 +128,28 @@ def test_wide_table(ff, gpu, B, Hq, Hkv, S, rule):
         assert pieces is None
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,D,S,lo", [
+    (3, 4, 2, 128, 20, 900),    # fewer groups than XCDs
+    (16, 16, 4, 128, 8, 0),     # 64 group slots of an XCD, all ranked together
+    (21, 6, 3, 64, 5, 0),       # groups that no XCD boundary divides
+    (33, 8, 2, 64, 30, 0),
+    (70, 2, 2, 64, 3, 0),       # more rows than lanes
+    (13, 16, 8, 256, 9, 0),
+    (30, 16, 8, 64, 2, 2400),   # rows alike: the order of the pieces
+    (9, 16, 4, 128, 8, -300),   # a call that stays whole
+])
+def test_rows_of_many_lengths(ff, gpu, B, Hq, Hkv, D, S, lo):
+    """Pieces dealt by their rows' lengths: each block's are done once, whatever the lengths and their order."""
+    rng = np.random.default_rng(1100 + B)
+    ctx = rng.integers(lo, 2500, size=B) if lo >= 0 else rng.integers(0, -lo, size=B)
+    ctx[B // 2] = 0 if lo <= 0 else lo
+    c, qn = _case(1100 + B, B, Hq, Hkv, D, [int(x) for x in ctx], S)
+    ref = O.paged_prefill_f64(qn, c.act, c.k_pool, c.v_pool, c.kv, c.block_table, c.ctx)
+    got, pieces = _pieces(ff, gpu, c, qn)
+    _check(got.reshape(ref.shape), ref, c.act, 2e-3)
+    assert (pieces >= 1).all() and (pieces > 1).any() == (lo >= 0)
+
+
 def test_split_prefill_reuses_scratch(ff, gpu):
     """Calls of different sizes in a row, their scratch handed on by the allocator with the former call's contents
     (test_wide_table has a workspace of all ones)."""
