@@ -105,6 +105,19 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
     const int end = min(begin + a.chunk, L);
     const int G = a.group;
 
+    const int32_t* table = a.block_table + static_cast<int64_t>(b) * a.max_blocks;
+    // the chunk's first page in this row and in one of the 256 rows around it, a thread each (see `once`)
+    int first = -1, other = -2;
+    if constexpr (CT == F32)
+    {
+        const int r = max(0, min(b - 128, a.batch - 256)) + tid;
+        if (begin < end)
+        {
+            first = table[begin >> 4];
+            if (r != b && r < a.batch) other = a.block_table[static_cast<int64_t>(r) * a.max_blocks + (begin >> 4)];
+        }
+    }
+
     float q[GP][8];
 #pragma unroll
     for (int g = 0; g < GP; ++g)
@@ -141,23 +154,20 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
     // token groups per trip gain another 1 % on the former and cost the latter 10 %: fewer waves fit.)  Any of the 256
     // rows around this one counts, a thread each: rows over two or ten prefixes in turn, no two neighbours alike, took 296
     // and 395 us where only the rows on either side were looked at, 194 and 357 now (all plain: 204 and 360).
-    const int32_t* table = a.block_table + static_cast<int64_t>(b) * a.max_blocks;
-    bool           once = CT == F32;
-    if constexpr (CT == F32)
-    {
-        if (begin < end)  // uniform over the workgroup
-        {
-            const int r = max(0, min(b - 128, a.batch - 256)) + tid;
-            const bool other = r != b && r < a.batch &&
-                               a.block_table[static_cast<int64_t>(r) * a.max_blocks + (begin >> 4)] == table[begin >> 4];
-            once = __syncthreads_or(other) == 0;
-        }
-    }
+    bool once = CT == F32;
+    if constexpr (CT == F32) once = __syncthreads_or(first == other) == 0;
 
     // U consecutive token groups per loop trip: their table entries, then all their K / V loads, go out before
     // any of them is used, so U times the bytes of one group are in flight per wave (none extra for the 16-head
     // groups, which already fill the registers).  The table entries of the next trip are requested while this trip's
     // tokens are computed.
+    // ALWAYS: tokens of no page, and lanes past the head, load too (from page 0, the token's first dims) and are left out
+    // where they would count.  Behind a branch the wait for the first group's K is, as far as the compiler can tell, one for
+    // nearly all loads, so that nothing is computed while they are on their way: with eight heads per KV head, where
+    // computing takes as long as loading, 32 rows of 512 to 4096 fp32 tokens at 64/8 heads 172.9 -> 165.7 us, 36 of 6600 to
+    // 12500 at head_dim 80 590 -> 555; with four heads of 128 dims 111.3 -> 112.1, with one at head_dim 72 (fp8) 36.4 -> 36.9.
+    constexpr bool ALWAYS = GP >= 8 || (DT == 0 && GP >= 4);
+    const int      stop = ALWAYS && a.num_blocks <= 0 ? begin : end;  // without a page there is nothing to load from
     auto stream = [&]<int U, bool NT>()
     {
         auto load_phys = [&](int base, int (&ph)[U])
@@ -171,7 +181,7 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
         };
         int phys[U];
         load_phys(begin, phys);
-        for (int base = begin; base < end; base += U * TPI)
+        for (int base = begin; base < stop; base += U * TPI)
         {
             bool   valid[U];
             size_t row[U];
@@ -188,10 +198,11 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
             for (int u = 0; u < U; ++u)
             {
                 ks[u] = vs[u] = 1.0f;
-                if (valid[u] && act)
+                if (ALWAYS || (valid[u] && act))
                 {
-                    load_row8<CT, NT>(a.k_cache, row[u], D, lane, kr[u]);
-                    load_row8<CT, NT>(a.v_cache, row[u], D, lane, vr[u]);
+                    const int ln = act ? lane : 0;
+                    load_row8<CT, NT>(a.k_cache, row[u], D, ln, kr[u]);
+                    load_row8<CT, NT>(a.v_cache, row[u], D, ln, vr[u]);
                     if constexpr (CT == I8)
                     {
                         ks[u] = a.k_scale[row[u]];
@@ -210,6 +221,9 @@ __global__ __launch_bounds__(256) void paged_decode_generic(DecodeArgs a)
             {
                 float k[8];
                 unpack8<CT>(kr[u], k);
+                if constexpr (ALWAYS && DT == 0)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) k[i] = act ? k[i] : 0.0f;
                 if constexpr (CT == I8 || CT == FP8)
                 {
                     const float sk = CT == I8 ? ks[u] : a.k_scale[kvh];

@@ -5,6 +5,7 @@ chunks (chunks of 256 tokens here, merged eight at a time).  Against the CPU che
 
 import math
 
+import numpy as np
 import pytest
 
 import cases
@@ -50,3 +51,20 @@ def test_vector_decode_merge(ff, gpu, kv, tol):
     """The same merge behind the vector kernel's other caches (head_dim 88)."""
     c = cases.make_case(740, 3, 12, 3, 88, [2047, 90, 3000], act="bf16", kv=kv, input_scale=1 / math.sqrt(88))
     _check(ff, gpu, c, tol)
+
+
+@pytest.mark.parametrize("act,kv,G,D", [("f32", "f32", 8, 128), ("f32", "f32", 5, 64), ("f32", "f32", 2, 80),
+                                        ("bf16", "bf16", 8, 88), ("bf16", "i8", 1, 40), ("f32", "f32", 3, 128)])
+def test_absent_pages_read_nothing(ff, gpu, act, kv, G, D):
+    """Page 0, which tokens of no page may load from, holds NaN and belongs to no row: no output shows it, a row without
+    any page is zero."""
+    c = cases.make_case(750 + D + G, 4, 2 * G, 2, D, [500, 37, 300, 64], act=act, kv=kv, input_scale=1 / math.sqrt(D))
+    c.block_table[c.block_table == 0] = -1
+    c.block_table[0, 5:9] = -1
+    c.block_table[0, 12] = c.num_blocks
+    c.block_table[3, :] = -1
+    if kv == "i8":
+        c.k_scale[0] = c.v_scale[0] = np.nan
+    else:
+        c.k_pool[0] = c.v_pool[0] = np.nan if kv == "f32" else 0x7FC0
+    _check(ff, gpu, c, 2e-2 if kv == "i8" else 2e-3 if kv == "bf16" else 1e-4)

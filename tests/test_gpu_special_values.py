@@ -124,6 +124,16 @@ def test_decode(ff, gpu, act, kv, kind, B, ctx):
         _check(_decode(ff, gpu, c, table), want, c, 2e-2 if kv in ("i8", "fp8") else 2e-3)
 
 
+@pytest.mark.parametrize("act,kv,kind", FORMS)
+@pytest.mark.parametrize("Hq,D", [(8, 88), (16, 128)])
+def test_vector_decode(ff, gpu, act, kv, kind, Hq, D):
+    """The vector kernel where its lanes past the head load like the others (a head dim of no instance of its own), and with
+    eight heads per KV head (fp32 pages)."""
+    c = cases.make_case(8300 + D, 3, Hq, 2, D, [300, 250, 90], act=act, kv=kv)
+    _plant(c, kind)
+    _check(_decode(ff, gpu, c, c.block_table), _expected(c), c, 2e-2 if kv in ("i8", "fp8") else 2e-3)
+
+
 @pytest.mark.parametrize("act,kv", [("bf16", "bf16"), ("f16", "f16"), ("bf16", "i8"), ("bf16", "fp8")])
 @pytest.mark.parametrize("kind", ["nan query", "nan key"])
 @pytest.mark.parametrize("B", [3, 40])
