@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -181,6 +182,19 @@ int decode_min_chunk(int cap_tokens)
 {
     int64_t c = ceil_div(ceil_div(cap_tokens, 64), kBlockSize) * kBlockSize;
     return static_cast<int>(c < 256 ? 256 : c);
+}
+
+// Most work items of a matrix-core decode: about 5 sqrt(pages) per row, and no fewer than 96.  A row's pieces are merged
+// one after the other by the waves of a workgroup per head, so with few long rows the resident workgroups' number of pieces
+// costs more there than it saves in the page loop; their number also went with the registers (head_dim 64: 1536 -> 2048
+// items, 2 rows of 12k to 24k tokens at 10/2 heads 38.2 -> 47.4 us).  All items -> these, us: that call 18.9; 1 row of 24k tokens
+// at 8/2 heads of 128 38.0 -> 18.2, at 32/8 26.3 -> 23.8; 4 rows of 4000 at 28/4 18.1 -> 15.5; 1 row of 120k at 10/2 heads
+// of 64 67.3 -> 30.7.  3 sqrt(pages) leaves too little in flight (1 row of 40k int8 tokens at 32/8 32.7 -> 37.5), and fewer
+// than 96 too short a page loop to hide its start.  Calls of 22 rows and more are never limited.
+int decode_most_items(int batch, int cap_tokens)
+{
+    const double per_row = std::max(96.0, 5.0 * std::sqrt(static_cast<double>(ceil_div(cap_tokens, kBlockSize))));
+    return static_cast<int>(std::min(per_row * batch, static_cast<double>(kMfmaMaxItems)));
 }
 
 // Grow the chunk while the grid still has >= 4096 work items at the row-length bound; long chunks cost fewer
@@ -555,6 +569,7 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
         a.pfx_share = plan.pfx_share;
     }
     a.items = fused_pfx ? plan.items : (mfma ? ffkv::decode_mfma_launch_items(a) : 0);
+    if (mfma && skip == 0) a.items = std::min(a.items, ffkv::decode_most_items(batch, cap));
 
     // workspace layout: MFMA kernel see mfma_layout, generic kernel [ml | acc] (none for single-chunk rows)
     ffkv::MfmaLayout lay{};

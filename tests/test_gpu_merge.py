@@ -33,3 +33,15 @@ def test_pieces_head_dims(ff, gpu, D, kv, act, B):
     c = cases.make_case(4100 + D + B, B, 6, 2, D, rng.integers(1, 900, size=B), act=act, kv=kv,
                         input_scale=1 / math.sqrt(D))
     _check(ff, gpu, c, 2e-3 if kv in ("bf16", "f16") else 2e-2)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,ctx,kv", [
+    (1, 10, 2, 64, 20000, "bf16"), (2, 10, 2, 64, 5900, "f16"), (3, 8, 2, 128, 5897, "bf16"),
+    (1, 32, 8, 128, 9000, "i8"), (21, 10, 2, 64, 1500, "bf16"), (22, 10, 2, 64, 1500, "bf16")])
+def test_few_long_rows(ff, gpu, B, Hq, Hkv, D, ctx, kv):
+    """Fewer work items than workgroups fit the chip, by the rows' pages: above and below the least of them per row (96, 369
+    pages), and where the rows are as many that it limits nothing."""
+    act = "f16" if kv == "f16" else "bf16"
+    c = cases.make_case(4300 + B + D, B, Hq, Hkv, D, [ctx - 17 * (b % 7) for b in range(B)], act=act, kv=kv,
+                        input_scale=1 / math.sqrt(D))
+    _check(ff, gpu, c, 2e-2 if kv == "i8" else 2e-3)
