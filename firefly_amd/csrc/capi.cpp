@@ -569,7 +569,6 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
         a.pfx_share = plan.pfx_share;
     }
     a.items = fused_pfx ? plan.items : (mfma ? ffkv::decode_mfma_launch_items(a) : 0);
-    if (mfma && skip == 0) a.items = std::min(a.items, ffkv::decode_most_items(batch, cap));
 
     // workspace layout: MFMA kernel see mfma_layout, generic kernel [ml | acc] (none for single-chunk rows)
     ffkv::MfmaLayout lay{};
@@ -586,6 +585,9 @@ int decode_impl(const void* q, void* out, int qo_dtype, const void* k_cache, con
         lay.acc = align256(parts * 2 * 4);
         need = lay.acc + parts * head_dim * 4;
     }
+
+    // (the workspace is asked for as before the bound, so that the sizes refused do not depend on it)
+    if (mfma && skip == 0) a.items = std::min(a.items, ffkv::decode_most_items(batch, cap));
 
     a.cap_tokens = cap;
     const bool  row = mfma && skip == 0 && ffkv::decode_use_row(a);  // writes no partials

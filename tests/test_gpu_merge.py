@@ -45,3 +45,21 @@ def test_few_long_rows(ff, gpu, B, Hq, Hkv, D, ctx, kv):
     c = cases.make_case(4300 + B + D, B, Hq, Hkv, D, [ctx - 17 * (b % 7) for b in range(B)], act=act, kv=kv,
                         input_scale=1 / math.sqrt(D))
     _check(ff, gpu, c, 2e-2 if kv == "i8" else 2e-3)
+
+
+def test_few_long_rows_workspace(ff, gpu):
+    """The bound on work items leaves the workspace's limit where it is without: one that only the bounded items' partials
+    would fit is refused."""
+    import torch
+
+    B, Hq, Hkv, D, blocks = 1, 10, 2, 64, 1250  # 5 sqrt(1250) = 176 of at least 1024 resident workgroups
+    q = torch.zeros((B, 1, Hq, D), dtype=torch.bfloat16, device=gpu)
+    k = torch.zeros((1, 16, Hkv, D), dtype=torch.bfloat16, device=gpu)
+    table = torch.full((B, blocks), -1, dtype=torch.int32, device=gpu)
+    ctx = torch.full((B,), 19999, dtype=torch.int32, device=gpu)
+    ws = torch.empty((176 + B + 8) * Hq * (D + 2) * 4 + 4096, dtype=torch.uint8, device=gpu)
+    with pytest.raises(ff.FFKVError):
+        ff.paged_attention(q, k, k, table, ctx, workspace=ws)
+    out = ff.paged_attention(q, k, k, table, ctx, workspace=ff.decode_workspace(B, Hq, D, blocks, device=gpu))
+    torch.cuda.synchronize()
+    assert not out.any()
